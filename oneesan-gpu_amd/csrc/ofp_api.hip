@@ -21,6 +21,7 @@
 
 #include "../../include/ofp.h"
 #include "ofp_exchange_impl.h"
+#include "ofp_glue.h"
 #include "ofp_internal.h"
 #include "ofp_pair_impl.h"
 
@@ -47,6 +48,9 @@ struct Sweep {
     bool fixed = false;        // buffers are slices of the library's static device array (no graphs)
     int row = -1;              // rows swept since the initial state; -1: state of unknown origin
     std::vector<hipEvent_t> seg_ev;  // timing events of row segments (ofp_row_sweep)
+    uint64_t* acc = nullptr;         // the k sums of a half-row solve's last step (zeroed with the state)
+    uint32_t* gscratch = nullptr;    // its scratch (states of more than 20 positions)
+    size_t gscratch_cap = 0;
     // pair passes: two more streams for the launches of one pass that may run
     // side by side (created on first use, not for the static sweep)
     hipStream_t par[2] = {};
@@ -101,6 +105,16 @@ struct ofp_ctx {
     } last_low;
     char* stage = nullptr;  // exchange buffer: plan tables and staging buckets, reused
     size_t stage_bytes = 0;
+    // half-row solves (ofp_glue_impl.h): the ballot and binomial tables (host copies
+    // and one device allocation, which also holds ofp_solve_static's sums) and the
+    // lists of open meanders, those of more than kBaseStrands made when first needed
+    glue::Ballot ballot;
+    uint32_t binom[kMaxW * 32] = {};
+    char* gdev = nullptr;
+    const glue::Ballot* dballot = nullptr;
+    const uint32_t* dbinom = nullptr;
+    uint64_t* static_acc = nullptr;
+    glue::Tables gtab[glue::kTableSets];
     void* scratch = nullptr;  // device address of the static state array on this device
     Sweep fixed;           // ofp_solve_static's state, inside that array
     std::string err;
@@ -218,8 +232,11 @@ void free_sweep(Sweep& s) {
     sweep_free(s, s.main);
     sweep_free(s, s.blk);
     sweep_free(s, s.mods_dev);
-    s.main = s.blk = s.mods_dev = nullptr;
-    s.main_cap = s.blk_cap = 0;
+    sweep_free(s, s.acc);
+    sweep_free(s, s.gscratch);
+    s.main = s.blk = s.mods_dev = s.gscratch = nullptr;
+    s.acc = nullptr;
+    s.main_cap = s.blk_cap = s.gscratch_cap = 0;
     s.mods_cap = 0;
     s.layout = -1;
 }
@@ -324,9 +341,14 @@ ofp_status ensure_state(ofp_ctx* c, Sweep& s, int n, const uint32_t* moduli, int
     }
     if (s.mods_cap < k) {
         sweep_free(s, s.mods_dev);
+        sweep_free(s, s.acc);
         s.mods_dev = nullptr;
-        s.mods_cap = std::max(k, 16);
-        OFP_HIP(c, sweep_alloc(s, (void**)&s.mods_dev, s.mods_cap * sizeof(uint32_t)), "allocate moduli");
+        s.acc = nullptr;
+        s.mods_cap = 0;
+        const int cap = std::max(k, 16);
+        OFP_HIP(c, sweep_alloc(s, (void**)&s.mods_dev, cap * sizeof(uint32_t)), "allocate moduli");
+        OFP_HIP(c, sweep_alloc(s, (void**)&s.acc, cap * sizeof(uint64_t)), "allocate sums");
+        s.mods_cap = cap;
     }
     s.mods.assign(moduli, moduli + k);
     // stream-ordered copy from pageable memory (staged by the runtime before returning)
@@ -637,10 +659,10 @@ ofp_status full_rows(ofp_ctx* c, Sweep& s, int rows, int* launches) {
 }
 
 // True when some cell of row r (of a sweep from the initial state) runs capped.
-bool row_capped(const ofp_ctx* c, const Sweep& s, int r) {
+bool row_capped(const ofp_ctx* c, const Sweep& s, int r, int p_lo = 1) {
     const int pct = cap_pct(c, s);
     if (pct <= 0 || r < 0 || s.layout != 1) return false;
-    for (int p = s.W - 1; p >= 1; --p)
+    for (int p = s.W - 1; p >= p_lo; --p)
         if (effective_cap(s.W, r, p, s.nblk, nullptr, pct)) return true;
     return false;
 }
@@ -648,11 +670,12 @@ bool row_capped(const ofp_ctx* c, const Sweep& s, int r) {
 // A row with capped cells (row r of a sweep from the initial state): each capped
 // cell alone, each run of uncapped cells as full-state cells, paired as in a
 // full row where pair passes apply.  (A pair pass is two consecutive full-state
-// cells, so the row computes what one launch per cell computes.)
-ofp_status enqueue_capped_row(ofp_ctx* c, Sweep& s, int r, int* launches) {
-    if (!pair_ready(c, s)) return enqueue_cells(c, s, s.W - 1, 1, false, launches, r);
+// cells, so the row computes what one launch per cell computes.)  p_lo > 1: only
+// the row's cells W-1..p_lo.
+ofp_status enqueue_capped_row(ofp_ctx* c, Sweep& s, int r, int* launches, int p_lo = 1) {
+    if (!pair_ready(c, s)) return enqueue_cells(c, s, s.W - 1, p_lo, false, launches, r);
     const int pct = cap_pct(c, s);
-    for (int p = s.W - 1; p >= 1;) {
+    for (int p = s.W - 1; p >= p_lo;) {
         const bool reads_blk = p != s.W - 1;
         if (effective_cap(s.W, r, p, s.nblk, nullptr, pct)) {
             ofp_status st = enqueue_cells(c, s, p, p, reads_blk, launches, r);
@@ -661,7 +684,7 @@ ofp_status enqueue_capped_row(ofp_ctx* c, Sweep& s, int r, int* launches) {
             continue;
         }
         int q = p;
-        while (q - 1 >= 1 && !effective_cap(s.W, r, q - 1, s.nblk, nullptr, pct)) --q;
+        while (q - 1 >= p_lo && !effective_cap(s.W, r, q - 1, s.nblk, nullptr, pct)) --q;
         ofp_status st = enqueue_pairs(c, s, p, q, reads_blk, launches);
         if (st) return st;
         p = q - 1;
@@ -676,10 +699,71 @@ struct RowTimes {
     int full_launches = 0, capped_launches = 0;
 };
 
+// The last step of a half-row solve (ofp_glue_impl.h) on s.stream.
+ofp_status enqueue_glue(ofp_ctx* c, Sweep& s, int* launches) {
+    const bool wide = s.W > 23 || c->index_bits == 64;
+    glue::GlueLaunch a{};
+    a.main = s.main;
+    a.blk = s.blk;
+    a.dp = wide ? c->dp64 : c->dp32;
+    a.ballot = c->dballot;
+    a.binom = c->dbinom;
+    a.acc = s.acc;
+    a.mods = s.mods_dev;
+    a.scratch = s.gscratch;
+    a.W = s.W;
+    a.K = s.Kp;
+    a.k = s.K;
+    a.center = (s.W & 1) ? (s.W - 1) / 2 : -1;
+    if (!a.mods)
+        for (int j = 0; j < s.K; ++j) a.mod[j] = s.mods[j];
+    const hipError_t e = glue::launch_glue(a, c->gtab, c->ballot, c->binom, wide, c->cus, s.gscratch_cap, s.main, s.stream,
+                                           launches);
+    return e == hipSuccess ? OFP_OK : hip_fail(c, e, "glue launch");
+}
+
+// Whether a whole solve of s, at its first row, runs half of its rows and glues
+// the middle frontier to its half turn: where height caps are on, that is where
+// only the answer word is read afterwards (with caps off every main word is final
+// after the last row), state-major, from four columns up (below, the caps of the
+// last two rows would reach the first half) to 24 (n = 23, the largest size with
+// reference residues).  Makes the lists of 19 strands and the scratch where the
+// width needs them; where those do not fit HBM the solve runs all rows.
+bool half_ready(ofp_ctx* c, Sweep& s) {
+    if (s.layout != 1 || cap_pct(c, s) <= 0 || s.row != 0 || s.W < 4 || s.W > glue::kSumStrands + 1 || !s.acc) return false;
+    if (s.W > glue::kBaseStrands + 1 && !c->gtab[1].mem) {
+        size_t fr = 0, tot = 0;
+        // 2 bytes per open meander with 19 crossings: 16 MB
+        if (s.fixed || hipMemGetInfo(&fr, &tot) != hipSuccess || ((size_t)32 << 20) + c->reserve > fr) return false;
+        if (glue::build_tables(c->ballot, c->dballot, glue::kTabStrands, glue::kTabStrands, &c->gtab[0], c->gtab[1],
+                               c->stream) != hipSuccess) {
+            (void)hipGetLastError();
+            return false;
+        }
+    }
+    const size_t need = glue::scratch_need(c->ballot, s.W, s.Kp);
+    if (need > s.gscratch_cap) {
+        if (s.fixed) return false;
+        sweep_free(s, s.gscratch);
+        s.gscratch = nullptr;
+        s.gscratch_cap = 0;
+        size_t fr = 0, tot = 0;
+        if (hipMemGetInfo(&fr, &tot) != hipSuccess || need + c->reserve > fr) return false;
+        if (sweep_alloc(s, (void**)&s.gscratch, need) != hipSuccess) {
+            (void)hipGetLastError();
+            s.gscratch = nullptr;
+            return false;
+        }
+        s.gscratch_cap = need;
+    }
+    return true;
+}
+
 // `rows` rows from the sweep's current row: rows with capped cells are launched
 // directly, runs of uncapped rows from the row graph.  With `times`, each run
-// is bracketed by events and the call waits for the last one.
-ofp_status run_rows(ofp_ctx* c, Sweep& s, int rows, int* launches, RowTimes* times = nullptr) {
+// is bracketed by events and the call waits for the last one.  half (rows = W, at
+// the first row, half_ready): half of the rows' cells and the glue.
+ofp_status run_rows(ofp_ctx* c, Sweep& s, int rows, int* launches, RowTimes* times = nullptr, bool half = false) {
     struct Seg {
         bool capped;
         int launches;
@@ -693,20 +777,25 @@ ofp_status run_rows(ofp_ctx* c, Sweep& s, int rows, int* launches, RowTimes* tim
         }
         return s.seg_ev[i];
     };
+    const int whole = half ? s.W / 2 : rows;
+    const int mid_lo = (s.W + 1) / 2;  // half, odd W: the middle row's cells W-1..mid_lo
     int done = 0;
-    while (done < rows) {
+    while (done < whole || (half && (s.W & 1) && done == whole)) {
         const int r = s.row >= 0 ? s.row + done : -1;
-        const bool capped = row_capped(c, s, r);
+        const bool part = done == whole;
+        const bool capped = row_capped(c, s, r, part ? mid_lo : 1);
         int n = 1;
-        if (!capped)
-            while (done + n < rows && !row_capped(c, s, r < 0 ? -1 : r + n)) ++n;
+        if (!capped && !part)
+            while (done + n < whole && !row_capped(c, s, r < 0 ? -1 : r + n)) ++n;
         if (times) {
             hipEvent_t e = event(2 * segs.size());
             if (!e) return fail(c, OFP_E_RUNTIME, "event create");
             OFP_HIP(c, hipEventRecord(e, s.stream), "event record");
         }
         int l = 0;
-        ofp_status st = capped ? enqueue_capped_row(c, s, r, &l) : full_rows(c, s, n, &l);
+        ofp_status st = part     ? enqueue_capped_row(c, s, r, &l, mid_lo)
+                        : capped ? enqueue_capped_row(c, s, r, &l)
+                                 : full_rows(c, s, n, &l);
         if (st) return st;
         if (times) {
             hipEvent_t e = event(2 * segs.size() + 1);
@@ -717,6 +806,8 @@ ofp_status run_rows(ofp_ctx* c, Sweep& s, int rows, int* launches, RowTimes* tim
         if (launches) *launches += l;
         done += n;
     }
+    if (half)
+        if (ofp_status st = enqueue_glue(c, s, launches)) return st;
     if (s.row >= 0) s.row += rows;
     if (times && !segs.empty()) {
         OFP_HIP(c, hipEventSynchronize(s.seg_ev[2 * segs.size() - 1]), "row sweep sync");
@@ -744,8 +835,9 @@ ofp_status init_state(ofp_ctx* c, Sweep& s) {
             "zero blocked state");
     s.row = 0;
     uint64_t start = dp_at(s.W - 1, 1);
-    hipError_t e = s.mods_dev ? launch_set_one(s.main, start, s.Kp, s.K, s.layout, s.mods_dev, s.stream)
-                              : launch_set_one_values(s.main, start, s.Kp, s.K, s.layout, s.mods.data(), s.stream);
+    hipError_t e = s.mods_dev
+                       ? launch_set_one(s.main, start, s.Kp, s.K, s.layout, s.mods_dev, s.acc, s.stream)
+                       : launch_set_one_values(s.main, start, s.Kp, s.K, s.layout, s.mods.data(), s.acc, s.stream);
     if (e != hipSuccess) return hip_fail(c, e, "init kernel");
     return OFP_OK;
 }
@@ -821,6 +913,10 @@ ofp_status read_main(ofp_ctx* c, Sweep& s, uint64_t index, uint32_t* out_k, int 
         return fail(c, OFP_E_ARG, "output holds " + std::to_string(capacity) + " residues, the state has " +
                                       std::to_string(s.K) + " moduli");
     OFP_HIP(c, hipStreamSynchronize(s.stream), "sync");
+    if (s.layout == 1) {  // the k residues of a state are contiguous
+        OFP_HIP(c, hipMemcpy(out_k, s.main + index * (uint64_t)s.Kp, (size_t)s.K * 4, hipMemcpyDeviceToHost), "read residues");
+        return OFP_OK;
+    }
     for (int j = 0; j < s.K; ++j)
         OFP_HIP(c, hipMemcpy(out_k + j, s.main + state_elem(s.layout, index, s.Kp, j), 4, hipMemcpyDeviceToHost),
                 "read residue");
@@ -873,6 +969,8 @@ ofp_status ofp_create(const ofp_config* cfg, ofp_ctx** out) {
         if (c->dpc64) (void)hipFree(c->dpc64);
         if (c->ct32) (void)hipFree(c->ct32);
         if (c->ct64) (void)hipFree(c->ct64);
+        for (glue::Tables& t : c->gtab) glue::free_tables(t);
+        if (c->gdev) (void)hipFree(c->gdev);
         if (c->ev0) (void)hipEventDestroy(c->ev0);
         if (c->ev1) (void)hipEventDestroy(c->ev1);
         if (c->stream) (void)hipStreamDestroy(c->stream);
@@ -931,6 +1029,19 @@ ofp_status ofp_create(const ofp_config* cfg, ofp_ctx** out) {
         return OFP_E_RUNTIME;
     }
     if (bad(hipMalloc(&c->ct64, bt64)) || bad(hipMemcpy(c->ct64, t64.data(), bt64, hipMemcpyHostToDevice)))
+        return OFP_E_RUNTIME;
+    glue::build_ballot(c->ballot);
+    for (int p = 0; p < kMaxW; ++p)
+        for (int q = 0; q < 32; ++q)
+            c->binom[p * 32 + q] = q == 0 ? 1 : (p == 0 ? 0 : c->binom[(p - 1) * 32 + q] + c->binom[(p - 1) * 32 + q - 1]);
+    const size_t bal = (sizeof(glue::Ballot) + 255) / 256 * 256, bin = (sizeof c->binom + 255) / 256 * 256;
+    if (bad(hipMalloc(&c->gdev, bal + bin + kMaxKC * sizeof(uint64_t)))) return OFP_E_RUNTIME;
+    c->dballot = reinterpret_cast<const glue::Ballot*>(c->gdev);
+    c->dbinom = reinterpret_cast<const uint32_t*>(c->gdev + bal);
+    c->static_acc = reinterpret_cast<uint64_t*>(c->gdev + bal + bin);
+    if (bad(hipMemcpy(c->gdev, &c->ballot, sizeof c->ballot, hipMemcpyHostToDevice)) ||
+        bad(hipMemcpy(c->gdev + bal, c->binom, sizeof c->binom, hipMemcpyHostToDevice)) ||
+        bad(glue::build_tables(c->ballot, c->dballot, 1, glue::kBaseStrands, nullptr, c->gtab[0], c->stream)))
         return OFP_E_RUNTIME;
     *out = c;
     return OFP_OK;
@@ -1040,15 +1151,13 @@ ofp_status ofp_prepare(ofp_ctx* c, int n, const uint32_t* moduli, int k) {
     return OFP_OK;
 }
 
-ofp_status ofp_row_sweep(ofp_ctx* c, int rows, ofp_stats* st) {
-    if (!c || rows < 0) return OFP_E_ARG;
+static ofp_status row_sweep(ofp_ctx* c, int rows, ofp_stats* st, bool half) {
     Sweep& s = c->st;
-    if (!s.main || s.layout != c->layout) return fail(c, OFP_E_ARG, "no prepared state");
     int launches = 0;
     auto t0 = std::chrono::steady_clock::now();
     OFP_HIP(c, hipEventRecord(c->ev0, s.stream), "event record");
     RowTimes times;
-    ofp_status r = run_rows(c, s, rows, &launches, &times);
+    ofp_status r = run_rows(c, s, rows, &launches, &times, half);
     if (r) return r;
     OFP_HIP(c, hipEventRecord(c->ev1, s.stream), "event record");
     OFP_HIP(c, hipEventSynchronize(c->ev1), "row sweep sync");
@@ -1069,6 +1178,12 @@ ofp_status ofp_row_sweep(ofp_ctx* c, int rows, ofp_stats* st) {
         st->transitions = (uint64_t)rows * (s.W - 1) * (s.nmain + s.nblk) * (uint64_t)s.K;
     }
     return OFP_OK;
+}
+
+ofp_status ofp_row_sweep(ofp_ctx* c, int rows, ofp_stats* st) {
+    if (!c || rows < 0) return OFP_E_ARG;
+    if (!c->st.main || c->st.layout != c->layout) return fail(c, OFP_E_ARG, "no prepared state");
+    return row_sweep(c, rows, st, false);
 }
 
 ofp_status ofp_read_main(ofp_ctx* c, uint64_t index, uint32_t* out, int capacity) {
@@ -1170,7 +1285,7 @@ ofp_status ofp_solve(ofp_ctx* c, int n, const uint32_t* moduli, int k, uint32_t*
         s = init_state(c, c->st);
         if (s) return s;
         ofp_stats rs{};
-        s = ofp_row_sweep(c, c->st.W, &rs);
+        s = row_sweep(c, c->st.W, &rs, half_ready(c, c->st));
         if (s) return s;
         s = read_main(c, c->st, 0, residues_out + off, sizes[i]);  // rank_full(R) = 0 (fullmate_dropN_batch.cu:508,514)
         if (s) return s;
@@ -1215,6 +1330,7 @@ ofp_status ofp_solve_static(ofp_ctx* c, int n, const uint32_t* moduli, int k, ui
     s.main_cap = mb;
     s.blk_cap = bb;
     s.mods_dev = nullptr;  // the start word takes the moduli by value
+    s.acc = c->static_acc;
     s.mods.assign(moduli, moduli + k);
     s.n = n;
     s.W = n + 1;
@@ -1226,7 +1342,7 @@ ofp_status ofp_solve_static(ofp_ctx* c, int n, const uint32_t* moduli, int k, ui
     ofp_status st = init_state(c, s);  // clears both arrays: they hold the last call's state
     if (st) return st;
     int launches = 0;
-    st = run_rows(c, s, s.W, &launches);
+    st = run_rows(c, s, s.W, &launches, nullptr, half_ready(c, s));
     if (st) return st;
     st = read_main(c, s, 0, residues_out, k);
     s.main = s.blk = nullptr;
@@ -2029,7 +2145,8 @@ ofp_status ofp_job_enqueue(ofp_job* j, int rows) {
     if (!j || rows < 0) return OFP_E_ARG;
     ofp_ctx* c = j->ctx;
     if (j->rows_enqueued + rows > j->sw.W) return fail(c, OFP_E_ARG, "job has only W rows");
-    ofp_status st = run_rows(c, j->sw, rows, nullptr);
+    const bool half = j->rows_enqueued == 0 && rows == j->sw.W && half_ready(c, j->sw);
+    ofp_status st = run_rows(c, j->sw, rows, nullptr, nullptr, half);
     if (st) return st;
     j->rows_enqueued += rows;
     OFP_HIP(c, hipEventRecord(j->done, j->sw.stream), "job event record");
@@ -2077,6 +2194,8 @@ void ofp_destroy(ofp_ctx* c) {
     if (c->dpc64) (void)hipFree(c->dpc64);
     if (c->ct32) (void)hipFree(c->ct32);
     if (c->ct64) (void)hipFree(c->ct64);
+    for (glue::Tables& t : c->gtab) glue::free_tables(t);
+    if (c->gdev) (void)hipFree(c->gdev);
     for (int i = 0; i < 3; ++i) {
         if (c->gstream[i]) (void)hipStreamDestroy(c->gstream[i]);
         if (c->gjoin[i]) (void)hipEventDestroy(c->gjoin[i]);

@@ -193,9 +193,10 @@ __global__ void fill_remote_kernel(uint32_t* main, uint64_t m0, uint64_t M, uint
 }
 
 __global__ void set_one_kernel(uint32_t* main, uint64_t index, int K, int k, int layout,
-                               const uint32_t* mods) {
+                               const uint32_t* mods, uint64_t* acc) {
     int j = threadIdx.x;
     if (j < k) main[state_elem(layout, index, K, j)] = 1u % mods[j];
+    if (j < k && acc) acc[j] = 0;
 }
 
 template <typename Idx, int KC>
@@ -313,25 +314,27 @@ hipError_t launch_fill_remote(uint32_t* main, uint64_t m0, uint64_t M, uint32_t*
 struct ModVals {
     uint32_t m[kMaxKC];
 };
-__global__ void set_one_values_kernel(uint32_t* main, uint64_t index, int K, int k, int layout, ModVals mods) {
+__global__ void set_one_values_kernel(uint32_t* main, uint64_t index, int K, int k, int layout, ModVals mods,
+                                      uint64_t* acc) {
     int j = threadIdx.x;
     if (j < k) main[state_elem(layout, index, K, j)] = 1u % mods.m[j];
+    if (j < k && acc) acc[j] = 0;
 }
 
 hipError_t launch_set_one_values(uint32_t* main, uint64_t index, int K, int k, int layout,
-                                 const uint32_t* mods_host, hipStream_t s) {
+                                 const uint32_t* mods_host, uint64_t* acc, hipStream_t s) {
     if (k < 1 || k > kMaxKC || K < k) return hipErrorInvalidValue;
     ModVals mv{};
     for (int j = 0; j < k; ++j) mv.m[j] = mods_host[j];
-    hipLaunchKernelGGL(set_one_values_kernel, dim3(1), dim3(64), 0, s, main, index, K, k, layout, mv);
+    hipLaunchKernelGGL(set_one_values_kernel, dim3(1), dim3(64), 0, s, main, index, K, k, layout, mv, acc);
     return hipGetLastError();
 }
 
 hipError_t launch_set_one(uint32_t* main, uint64_t index, int K, int k, int layout,
-                          const uint32_t* mods_dev, hipStream_t s) {
+                          const uint32_t* mods_dev, uint64_t* acc, hipStream_t s) {
     if (k < 1 || k > 1024 || K < k) return hipErrorInvalidValue;
     hipLaunchKernelGGL(set_one_kernel, dim3(1), dim3(((k + 63) / 64) * 64), 0, s, main, index, K, k,
-                       layout, mods_dev);
+                       layout, mods_dev, acc);
     return hipGetLastError();
 }
 
