@@ -157,11 +157,13 @@ ofp_status ofp_time_cells(ofp_ctx* ctx, float* ms_out, int* kind_out, int capaci
  * place, in up to five launches (one per window height change that has
  * classes; the three that read other classes side by side, then the other
  * two), so every word is read and written once per two cells instead of once
- * per cell.  Height-capped cells still run one launch per cell.  32-bit and
+ * per cell.  Height-capped cells pair up likewise, over the classes within the
+ * cap.  32-bit and
  * 64-bit ranks (n >= 23) alike; the static solve (ofp_solve_static) runs the
  * launches one after another.  Results do not depend on it.
- * mode: 0 = off, 1 = on (the default), 2..16 (even) = on with at most that
- * many moduli per launch (default 16).  Walking down a row, cells p and p-1 run
+ * mode: 0 = off, 1 = on, 2..16 (even) = on with at most that many moduli per
+ * launch (default 16).  A context on which it was never called runs pair passes
+ * where a launch covers 2^23 words or more (n >= 17) and single cells below.  Walking down a row, cells p and p-1 run
  * as one pair pass when bit p of cell_mask is set (~0u: everywhere), else cell
  * p runs alone; 0 = the library's default (pairs except over cells 4 and 3;
  * the autotuner sets it per size).  Bits 8..9

@@ -74,9 +74,10 @@ struct ofp_ctx {
     void* dp64 = nullptr;  // packed uint64 height table
     void* dpc32 = nullptr; // packed capped tables, caps 1..kMaxCap (uint32, uint64)
     void* dpc64 = nullptr;
-    void* ct32 = nullptr;  // pair-pass class tables, every (p, d) (32-bit ranks)
+    void* ct32 = nullptr;  // pair-pass class tables, every (cap, p, d) (32-bit ranks)
     void* ct64 = nullptr;  // the same with 64-bit entries (n >= 23, or 64-bit ranks forced)
-    int pair_rows = 1;     // 1: full-state rows run as pair passes (two cells per pass, in place)
+    int pair_rows = -1;    // cells as pair passes (two cells per pass, in place): 1 yes, 0 no, -1 where the
+                           // launch covers kPairWords words
     int pair_kc = kMaxKC;  // moduli per pair-pass launch (even, <= 16)
     uint32_t pair_mask = 0;  // bit p: cells p and p-1 run as one pair pass; 0: the library's default
     int pair_variant = 0;    // pair-kernel variant (PairLaunch::variant)
@@ -310,7 +311,7 @@ struct Carve {
 // Whether n in the context's settings runs its full rows as pair passes: pair
 // mode on, state-major layout, at least two cells (32-bit ranks for n <= 22,
 // 64-bit above or when forced).
-bool pairs_apply(const ofp_ctx* c, int n) { return c->pair_rows && c->layout == 1 && n >= 2; }
+bool pairs_apply(const ofp_ctx* c, int n) { return c->pair_rows != 0 && c->layout == 1 && n >= 2; }
 
 ofp_status ensure_state(ofp_ctx* c, Sweep& s, int n, const uint32_t* moduli, int k) {
     uint64_t nm, nb;
@@ -519,16 +520,104 @@ ofp_status pass_streams(ofp_ctx* c, Sweep& s) {
     return OFP_OK;
 }
 
-ofp_status enqueue_pairs(ofp_ctx* c, Sweep& s, int p_hi, int p_lo, bool first_reads_blk, int* launches,
-                         hipEvent_t* cell_ev = nullptr, int* cell_kind = nullptr) {
+// Words from which two cells run as one pair pass unless asked otherwise: a pass is
+// up to five launches, whose fixed times outweigh the bytes saved on few words.
+// Whole solves, cells alone against passes: n=16 (5.7e6 words) 3.19 against 4.06 ms at
+// one modulus, 7.85 against 8.33 at eight; n=17 (1.6e7) 6.82 against 6.65 and 24.5
+// against 22.9; n=14 (7e5) 1.05 against 1.90, 2.29 against 3.52.
+constexpr uint64_t kPairWords = 1ull << 23;
+// State bytes a pass covers from which its launches run side by side on three
+// streams.  Below, the fork and join cost more than the overlap gives: the capped
+// rows of an n=18 solve of one modulus (at most 177 MB) 5.17 ms with them, 4.17
+// without; above, an n=17 solve of eight (507 MB) 22.4 against 22.9 ms.
+constexpr uint64_t kParallelBytes = 384ull << 20;
+
+// Words of the cells' launches at height cap `cap` (0: the whole state).
+uint64_t covered_words(const Sweep& s, int cap) {
+    if (!cap) return s.nmain + s.nblk;
+    return (uint64_t)((double)(s.nmain + s.nblk) * (double)capped_blocked_count(s.W, cap) / (double)s.nblk);
+}
+
+// Whether cells p and p-1 run as one pair pass in a walk down to cell p_lo, at
+// height cap `cap`.
+bool pair_at(const ofp_ctx* c, const Sweep& s, int p, int p_lo, int cap) {
+    const uint32_t mask = c->pair_mask ? c->pair_mask : default_pair_mask(std::min(s.K, c->pair_kc));
+    return p - 1 >= p_lo && p >= 2 && ((mask >> p) & 1u) && (c->pair_rows > 0 || covered_words(s, cap) >= kPairWords);
+}
+
+// One pair pass over cells p and p-1 (cap > 0: over the classes at heights <= cap).
+ofp_status enqueue_pair(ofp_ctx* c, Sweep& s, int p, bool reads_blk, int cap, int* launches) {
     const int W = s.W;
     const bool wide = s.W > 23 || c->index_bits == 64;
     const size_t tb = class_table_bytes(wide);
-    const uint32_t mask = c->pair_mask ? c->pair_mask : default_pair_mask(std::min(s.K, c->pair_kc));
+    const bool par = !s.fixed && covered_words(s, cap) * (uint64_t)s.Kp * 4 >= kParallelBytes;
+    for (int off = 0; off < s.Kp; off += c->pair_kc) {
+        const int kc = std::min(c->pair_kc, s.Kp - off);
+        static const int kOrder[5] = {-1, 0, 1, -2, 2};
+        // The readers (d = -1, 0, 1) never read each other's changed words and
+        // the d = -2, 2 classes read only their own, so each of the two groups
+        // of launches runs side by side on three streams (fork before, join
+        // after): their ramp-ups and tails overlap.
+        if (par)
+            if (ofp_status f = pass_streams(c, s)) return f;
+        auto fork = [&]() -> ofp_status {
+            if (!par) return OFP_OK;
+            OFP_HIP(c, hipEventRecord(s.pfork, s.stream), "pair pass fork");
+            for (int q = 0; q < 2; ++q) OFP_HIP(c, hipStreamWaitEvent(s.par[q], s.pfork, 0), "pair pass fork");
+            return OFP_OK;
+        };
+        auto join = [&]() -> ofp_status {
+            if (!par) return OFP_OK;
+            for (int q = 0; q < 2; ++q) {
+                OFP_HIP(c, hipEventRecord(s.pjoin[q], s.par[q]), "pair pass join");
+                OFP_HIP(c, hipStreamWaitEvent(s.stream, s.pjoin[q], 0), "pair pass join");
+            }
+            return OFP_OK;
+        };
+        for (int di = 0; di < 5; ++di) {
+            const int d = kOrder[di];
+            if (di == 3)
+                if (ofp_status f = join()) return f;
+            if (di == 0 || di == 3)
+                if (ofp_status f = fork()) return f;
+            const uint64_t cnt = pair_class_count(W, p, d, cap);
+            if (!cnt) continue;
+            pair::PairLaunch a{};
+            a.main_in = s.main;
+            a.blk_in = s.blk;
+            a.main_out = s.main;
+            a.blk_out = s.blk;
+            a.dp = wide ? c->dp64 : c->dp32;
+            a.ct = static_cast<const char*>(wide ? c->ct64 : c->ct32) + tb * (size_t)((cap * kMaxW + p) * 7 + d + 3);
+            a.classes = cnt;
+            a.W = W;
+            a.p = p;
+            a.d = d;
+            a.read_blk = reads_blk ? 1 : 0;
+            a.cap = cap;
+            a.K = s.Kp;
+            a.off = off;
+            a.kc = kc;
+            // lanes past the k moduli (stride padding) compute with a valid modulus
+            for (int jj = 0; jj < kc; ++jj) a.mod[jj] = s.mods[off + jj < s.K ? off + jj : 0];
+            a.xcd_shift = piece_shift(c->xcd_shift, cnt, c->threads);
+            a.variant = c->pair_variant;
+            hipStream_t ls = !par ? s.stream : (d == -1 || d == -2) ? s.par[0] : (d == 1 ? s.par[1] : s.stream);
+            hipError_t e = launch_pair(a, wide, c->threads, grid_blocks(c, cnt), ls);
+            if (e != hipSuccess) return hip_fail(c, e, "pair pass launch");
+            if (launches) ++*launches;
+        }
+        if (ofp_status f = join()) return f;
+    }
+    return OFP_OK;
+}
+
+ofp_status enqueue_pairs(ofp_ctx* c, Sweep& s, int p_hi, int p_lo, bool first_reads_blk, int* launches,
+                         hipEvent_t* cell_ev = nullptr, int* cell_kind = nullptr) {
     for (int p = p_hi; p >= p_lo;) {
         const int slot = p_hi - p;
         const bool reads_blk = p == p_hi ? first_reads_blk : true;
-        if (!(p - 1 >= p_lo && p >= 2 && ((mask >> p) & 1u))) {
+        if (!pair_at(c, s, p, p_lo, 0)) {
             ofp_status st = enqueue_cells(c, s, p, p, reads_blk, launches, -1, cell_ev ? cell_ev + 2 * slot : nullptr,
                                           cell_kind ? cell_kind + slot : nullptr);
             if (st) return st;
@@ -536,67 +625,7 @@ ofp_status enqueue_pairs(ofp_ctx* c, Sweep& s, int p_hi, int p_lo, bool first_re
             continue;
         }
         if (cell_ev) OFP_HIP(c, hipEventRecord(cell_ev[2 * slot], s.stream), "event record");
-        for (int off = 0; off < s.Kp; off += c->pair_kc) {
-            const int kc = std::min(c->pair_kc, s.Kp - off);
-            static const int kOrder[7] = {-1, 0, 1, -3, -2, 2, 3};
-            // The readers (d = -1, 0, 1) never read each other's changed words and
-            // the d = -2, 2 classes read only their own, so each of the two groups
-            // of launches runs side by side on three streams (fork before, join
-            // after): their ramp-ups and tails overlap.
-            const bool par = !s.fixed;
-            if (par)
-                if (ofp_status f = pass_streams(c, s)) return f;
-            auto fork = [&]() -> ofp_status {
-                if (!par) return OFP_OK;
-                OFP_HIP(c, hipEventRecord(s.pfork, s.stream), "pair pass fork");
-                for (int q = 0; q < 2; ++q) OFP_HIP(c, hipStreamWaitEvent(s.par[q], s.pfork, 0), "pair pass fork");
-                return OFP_OK;
-            };
-            auto join = [&]() -> ofp_status {
-                if (!par) return OFP_OK;
-                for (int q = 0; q < 2; ++q) {
-                    OFP_HIP(c, hipEventRecord(s.pjoin[q], s.par[q]), "pair pass join");
-                    OFP_HIP(c, hipStreamWaitEvent(s.stream, s.pjoin[q], 0), "pair pass join");
-                }
-                return OFP_OK;
-            };
-            for (int di = 0; di < 7; ++di) {
-                const int d = kOrder[di];
-                if (di == 3)
-                    if (ofp_status f = join()) return f;
-                if (di == 0 || di == 4)
-                    if (ofp_status f = fork()) return f;
-                // d = -3 / +3: the class is one word, RRR or LLL, which neither cell
-                // changes (no target at (p, p-1) nor at (p-1, p-2)): nothing to do
-                if (d == -3 || d == 3) continue;
-                const uint64_t cnt = pair_class_count(W, p, d);
-                if (!cnt) continue;
-                pair::PairLaunch a{};
-                a.main_in = s.main;
-                a.blk_in = s.blk;
-                a.main_out = s.main;
-                a.blk_out = s.blk;
-                a.dp = wide ? c->dp64 : c->dp32;
-                a.ct = static_cast<const char*>(wide ? c->ct64 : c->ct32) + tb * (size_t)(p * 7 + d + 3);
-                a.classes = cnt;
-                a.W = W;
-                a.p = p;
-                a.d = d;
-                a.read_blk = reads_blk ? 1 : 0;
-                a.K = s.Kp;
-                a.off = off;
-                a.kc = kc;
-                // lanes past the k moduli (stride padding) compute with a valid modulus
-                for (int jj = 0; jj < kc; ++jj) a.mod[jj] = s.mods[off + jj < s.K ? off + jj : 0];
-                a.xcd_shift = piece_shift(c->xcd_shift, cnt, c->threads);
-                a.variant = c->pair_variant;
-                hipStream_t ls = !par ? s.stream : (d == -1 || d == -2) ? s.par[0] : (d == 1 ? s.par[1] : s.stream);
-                hipError_t e = launch_pair(a, wide, c->threads, grid_blocks(c, cnt), ls);
-                if (e != hipSuccess) return hip_fail(c, e, "pair pass launch");
-                if (launches) ++*launches;
-            }
-            if (ofp_status f = join()) return f;
-        }
+        if (ofp_status st = enqueue_pair(c, s, p, reads_blk, 0, launches)) return st;
         if (cell_ev) {
             OFP_HIP(c, hipEventRecord(cell_ev[2 * slot + 1], s.stream), "event record");
             OFP_HIP(c, hipEventRecord(cell_ev[2 * (slot + 1)], s.stream), "event record");
@@ -667,27 +696,28 @@ bool row_capped(const ofp_ctx* c, const Sweep& s, int r, int p_lo = 1) {
     return false;
 }
 
-// A row with capped cells (row r of a sweep from the initial state): each capped
-// cell alone, each run of uncapped cells as full-state cells, paired as in a
-// full row where pair passes apply.  (A pair pass is two consecutive full-state
-// cells, so the row computes what one launch per cell computes.)  p_lo > 1: only
-// the row's cells W-1..p_lo.
+// A row with capped cells (row r of a sweep from the initial state), paired as a
+// full row is where pair passes apply.  Two capped cells run as a pair pass over the
+// classes whose P' and S' stay at the greater of their caps: those hold every
+// blocked word the two cells sweep, and a class left out holds only words above the
+// cap.  (Cells swept whole where a cap would do compute what the capped ones do and
+// values that nothing reads.)  p_lo > 1: only the row's cells W-1..p_lo.
 ofp_status enqueue_capped_row(ofp_ctx* c, Sweep& s, int r, int* launches, int p_lo = 1) {
     if (!pair_ready(c, s)) return enqueue_cells(c, s, s.W - 1, p_lo, false, launches, r);
     const int pct = cap_pct(c, s);
     for (int p = s.W - 1; p >= p_lo;) {
         const bool reads_blk = p != s.W - 1;
-        if (effective_cap(s.W, r, p, s.nblk, nullptr, pct)) {
-            ofp_status st = enqueue_cells(c, s, p, p, reads_blk, launches, r);
-            if (st) return st;
+        ofp_status st;
+        const int c0 = effective_cap(s.W, r, p, s.nblk, nullptr, pct), c1 = effective_cap(s.W, r, p - 1, s.nblk, nullptr, pct);
+        const int cap = c0 && c1 && std::max(c0, c1) <= kPairCaps ? std::max(c0, c1) : 0;
+        if (pair_at(c, s, p, p_lo, cap)) {
+            st = enqueue_pair(c, s, p, reads_blk, cap, launches);
+            p -= 2;
+        } else {
+            st = enqueue_cells(c, s, p, p, reads_blk, launches, r);
             --p;
-            continue;
         }
-        int q = p;
-        while (q - 1 >= p_lo && !effective_cap(s.W, r, q - 1, s.nblk, nullptr, pct)) --q;
-        ofp_status st = enqueue_pairs(c, s, p, q, reads_blk, launches);
         if (st) return st;
-        p = q - 1;
     }
     return OFP_OK;
 }
@@ -1014,21 +1044,9 @@ ofp_status ofp_create(const ofp_config* cfg, ofp_ctx** out) {
     if (bad(hipMemcpy(c->dpc32, c32.data(), bc32, hipMemcpyHostToDevice)) ||
         bad(hipMemcpy(c->dpc64, c64.data(), bc64, hipMemcpyHostToDevice)))
         return OFP_E_RUNTIME;
-    std::vector<unsigned char> t32(class_table_bytes(false) * kMaxW * 7);
-    const size_t bt32 = pack_class_tables(false, t32.data(), t32.size());
-    if (!bt32) {
-        (void)bad(hipErrorInvalidValue);
-        return OFP_E_RUNTIME;
-    }
-    if (bad(hipMalloc(&c->ct32, bt32)) || bad(hipMemcpy(c->ct32, t32.data(), bt32, hipMemcpyHostToDevice)))
-        return OFP_E_RUNTIME;
-    std::vector<unsigned char> t64(class_table_bytes(true) * kMaxW * 7);
-    const size_t bt64 = pack_class_tables(true, t64.data(), t64.size());
-    if (!bt64) {
-        (void)bad(hipErrorInvalidValue);
-        return OFP_E_RUNTIME;
-    }
-    if (bad(hipMalloc(&c->ct64, bt64)) || bad(hipMemcpy(c->ct64, t64.data(), bt64, hipMemcpyHostToDevice)))
+    const size_t tables = (size_t)(kPairCaps + 1) * kMaxW * 7;
+    if (bad(hipMalloc(&c->ct32, tables * class_table_bytes(false))) || bad(hipMalloc(&c->ct64, tables * class_table_bytes(true))) ||
+        bad(launch_class_tables(false, c->ct32, c->stream)) || bad(launch_class_tables(true, c->ct64, c->stream)))
         return OFP_E_RUNTIME;
     glue::build_ballot(c->ballot);
     for (int p = 0; p < kMaxW; ++p)
@@ -1228,7 +1246,7 @@ ofp_status ofp_set_pair_passes(ofp_ctx* c, int mode, uint32_t cell_mask) {
         return fail(c, OFP_E_ARG, "pair passes: 0 (off), 1 (on) or an even moduli count per launch up to 16");
     if (variant != c->pair_variant) drop_graph(c->st);
     c->pair_variant = variant;
-    const int on = mode > 0 ? 1 : 0;
+    const int on = mode > 0 ? 1 : 0;  // asked for: at every size
     if (on != c->pair_rows) drop_graph(c->st);
     c->pair_rows = on;
     c->pair_kc = mode > 1 ? mode : kMaxKC;

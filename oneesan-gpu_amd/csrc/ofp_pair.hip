@@ -9,8 +9,6 @@
 // still hold their values from before the pass when it reads them (launch
 // order d = -1, 0, 1, then -2, 2), so the launches need no atomics and no
 // second copy of the state.
-#include <cstring>
-
 #include "ofp_pair_impl.h"
 
 namespace ofp {
@@ -26,7 +24,8 @@ __device__ void load_rows(T* dst, const T* src) {
 
 // MB: workgroups of 256 per CU the register allocation must allow (2: at most
 // 256 VGPRs, no spills at 14 moduli; 3: at most 168, with spills).
-template <int KC, typename Idx, int D, int GF, int MB>
+// Capped: the classes of a height-capped pass (a.cap).
+template <int KC, typename Idx, int D, int GF, int MB, bool Capped>
 __global__ __launch_bounds__(256, MB) void pair_kernel(pair::PairLaunch a) {
     constexpr int C = LdsCols<Idx>::value;
     __shared__ Quad<Idx> tab[kLdsRows][C];
@@ -41,32 +40,32 @@ __global__ __launch_bounds__(256, MB) void pair_kernel(pair::PairLaunch a) {
     for (uint64_t t = sc.slot; t < sc.count; t += sc.nx) {
         const uint64_t c = sc.chunk(t) * blockDim.x + threadIdx.x;
         if (c < a.classes) {
-            const pair::Class<Idx> k = pair::decode_class<Idx>(T, ctab, a.W, a.p, c);
+            const pair::Class<Idx> k = Capped ? pair::decode_class_capped<Idx>(T, ctab, a.W, a.p, D, c)
+                                              : pair::decode_class<Idx>(T, ctab, a.W, a.p, c);
             pair::pair_body<KC, Idx, D, GF>(a, T, k, io);
         }
     }
 }
 
-template <int KC, typename Idx, int GF, int MB>
+// The classes with d = -3, 3 change nothing and get no launch.
+template <int KC, typename Idx, int GF, int MB, bool Capped = false>
 hipError_t launch_d(const pair::PairLaunch& a, int threads, int blocks, hipStream_t s) {
     switch (a.d) {
-        case -3: hipLaunchKernelGGL((pair_kernel<KC, Idx, -3, GF, MB>), dim3(blocks), dim3(threads), 0, s, a); break;
-        case -2: hipLaunchKernelGGL((pair_kernel<KC, Idx, -2, GF, MB>), dim3(blocks), dim3(threads), 0, s, a); break;
-        case -1: hipLaunchKernelGGL((pair_kernel<KC, Idx, -1, GF, MB>), dim3(blocks), dim3(threads), 0, s, a); break;
-        case 0: hipLaunchKernelGGL((pair_kernel<KC, Idx, 0, GF, MB>), dim3(blocks), dim3(threads), 0, s, a); break;
-        case 1: hipLaunchKernelGGL((pair_kernel<KC, Idx, 1, GF, MB>), dim3(blocks), dim3(threads), 0, s, a); break;
-        case 2: hipLaunchKernelGGL((pair_kernel<KC, Idx, 2, GF, MB>), dim3(blocks), dim3(threads), 0, s, a); break;
-        case 3: hipLaunchKernelGGL((pair_kernel<KC, Idx, 3, GF, MB>), dim3(blocks), dim3(threads), 0, s, a); break;
+#define OFP_D(d) \
+    case d: hipLaunchKernelGGL((pair_kernel<KC, Idx, d, GF, MB, Capped>), dim3(blocks), dim3(threads), 0, s, a); break;
+        OFP_D(-2) OFP_D(-1) OFP_D(0) OFP_D(1) OFP_D(2)
+#undef OFP_D
         default: return hipErrorInvalidValue;
     }
     return hipGetLastError();
 }
 
 // Pair-kernel variant (PairLaunch::variant): bit 0 = gathers first, bit 1 = the
-// three-workgroups-per-CU register budget; only the 14- and 16-moduli kernels
-// carry the variants (the others run variant 0).
+// three-workgroups-per-CU register budget; only the whole-state 14- and 16-moduli
+// kernels carry the variants (the others run variant 0).
 template <int KC, typename Idx>
 hipError_t launch_gf(const pair::PairLaunch& a, int threads, int blocks, hipStream_t s) {
+    if (a.cap > 0) return launch_d<KC, Idx, 0, 2, true>(a, threads, blocks, s);
     if constexpr (KC >= 14) {
         switch (a.variant & 3) {
             case 1: return launch_d<KC, Idx, 1, 2>(a, threads, blocks, s);
@@ -78,49 +77,64 @@ hipError_t launch_gf(const pair::PairLaunch& a, int threads, int blocks, hipStre
     return launch_d<KC, Idx, 0, 2>(a, threads, blocks, s);
 }
 
-}  // namespace
-
-size_t pack_class_tables(bool wide, void* out, size_t cap) {
-    uint64_t d0[kDpRows][kDpCols];
-    build_height_table(d0);
-    const size_t one = (wide ? sizeof(Pair<uint64_t>) : sizeof(Pair<uint32_t>)) * kLdsRows *
-                       (wide ? LdsCols<uint64_t>::value : LdsCols<uint32_t>::value);
-    const size_t bytes = one * kMaxW * 7;
-    if (cap < bytes) return 0;
-    char* o = static_cast<char*>(out);
-    for (int p = 0; p < kMaxW; ++p)
-        for (int d = -3; d <= 3; ++d) {
-            char* dst = o + one * (size_t)(p * 7 + d + 3);
-            if (wide) {
-                static Pair<uint64_t> t[kDpRows][LdsCols<uint64_t>::value];
-                pair::pack_class_table<uint64_t, LdsCols<uint64_t>::value>(d0, p, d, t);
-                std::memcpy(dst, t, one);
-            } else {
-                static Pair<uint32_t> t[kDpRows][LdsCols<uint32_t>::value];
-                pair::pack_class_table<uint32_t, LdsCols<uint32_t>::value>(d0, p, d, t);
-                std::memcpy(dst, t, one);
-            }
-        }
-    return bytes;
+// Class tables of every (cap, p, d), cap 0 = none, one wave each (lane = height):
+// the height table's rows from the bottom up to p-2, then the class counts above p
+// (pair::build_class_table with the cap), packed as pair::pack_class_table does.
+template <typename Idx>
+__global__ __launch_bounds__(64) void class_tables_kernel(Pair<Idx>* out) {
+    constexpr int C = LdsCols<Idx>::value;
+    const int d = (int)(blockIdx.x % 7) - 3, p = (int)(blockIdx.x / 7) % kMaxW, cap = (int)(blockIdx.x / 7) / kMaxW;
+    const int h = (int)threadIdx.x, top = cap > 0 ? cap : kDpCols - 1;
+    const bool in = h <= top;
+    Pair<Idx>* t = out + (size_t)blockIdx.x * kLdsRows * C;
+    const auto at = [&](uint64_t v, int q) -> uint64_t {  // the value at height q, 0 outside 0..top
+        const uint64_t x = __shfl(v, q & 63);
+        return q >= 0 && q <= top ? x : 0;
+    };
+    const auto put = [&](int row, uint64_t v) {
+        const uint64_t below = at(v, h - 1);
+        if (h < C) t[row * C + h] = Pair<Idx>{(Idx)v, (Idx)(v + below)};
+    };
+    uint64_t v = h == 0 ? 1 : 0;  // the height table's row w
+    for (int w = 0; w < p - 2; ++w) {
+        put(w, cap > 0 ? v : 0);
+        const uint64_t dn = at(v, h - 1), up = at(v, h + 1);
+        v = in ? v + dn + up : 0;
+    }
+    v = p >= 2 ? at(v, h + d) : 0;  // row p-2 at height h + d
+    v = in ? v : 0;
+    for (int m = p < 2 ? 0 : p - 2; m <= p && m < kLdsRows; ++m) put(m, 0);
+    for (int m = p + 1; m < kLdsRows; ++m) {
+        put(m, v);
+        const uint64_t dn = at(v, h - 1), up = at(v, h + 1);
+        v = in ? v + dn + up : 0;
+    }
 }
+
+}  // namespace
 
 size_t class_table_bytes(bool wide) {
     return (wide ? sizeof(Pair<uint64_t>) * LdsCols<uint64_t>::value : sizeof(Pair<uint32_t>) * LdsCols<uint32_t>::value) *
            kLdsRows;
 }
 
-uint64_t pair_class_count(int W, int p, int d) {
-    static uint64_t d0[kDpRows][kDpCols];
-    static bool ready = false;
-    if (!ready) {
-        build_height_table(d0);
-        ready = true;
-    }
-    return pair::class_count(d0, W, p, d);
+hipError_t launch_class_tables(bool wide, void* out, hipStream_t s) {
+    const dim3 grid((kPairCaps + 1) * kMaxW * 7);
+    if (wide) hipLaunchKernelGGL((class_tables_kernel<uint64_t>), grid, dim3(64), 0, s, (Pair<uint64_t>*)out);
+    else hipLaunchKernelGGL((class_tables_kernel<uint32_t>), grid, dim3(64), 0, s, (Pair<uint32_t>*)out);
+    return hipGetLastError();
+}
+
+uint64_t pair_class_count(int W, int p, int d, int cap) {
+    uint64_t d0[kDpRows][kDpCols];
+    if (cap > 0) build_capped_table(cap, d0);
+    else build_height_table(d0);
+    return pair::class_count(d0, W, p, d, cap);
 }
 
 hipError_t launch_pair(const pair::PairLaunch& a, bool wide, int threads, int blocks, hipStream_t s) {
-    if (a.p < 2 || a.p > a.W - 1 || a.d < -3 || a.d > 3 || a.kc < 1 || a.off + a.kc > a.K) return hipErrorInvalidValue;
+    if (a.p < 2 || a.p > a.W - 1 || a.d < -3 || a.d > 3 || a.kc < 1 || a.off + a.kc > a.K || a.cap < 0 || a.cap > kPairCaps)
+        return hipErrorInvalidValue;
     if (wide) {
         switch (a.kc) {
             case 1: return launch_gf<1, uint64_t>(a, threads, blocks, s);

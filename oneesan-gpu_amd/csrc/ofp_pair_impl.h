@@ -138,10 +138,11 @@ struct PairLaunch {
     uint32_t* main_out;
     uint32_t* blk_out;
     const void* dp;    // packed height table (cell::Quad, kDpRows x kDpCols)
-    const void* ct;    // class table of (p, d): cell::Pair, kDpRows x kDpCols
+    const void* ct;    // class table of (p, d, cap): cell::Pair, kLdsRows x LdsCols
     uint64_t classes;  // classes of (p, d)
     int W, p, d;
     int read_blk;      // blocked input of cell p is valid (false at the first cell of a row)
+    int cap;           // > 0: only the classes whose P' and S' stay at heights <= cap
     int K, off, kc;    // interleave stride, first modulus, moduli in this launch
     int xcd_shift;
     int variant;        // kernel variant: bit 0 = gathers first (pair_body's GF), bit 1 = tighter registers
@@ -183,6 +184,28 @@ OFP_HD Class<Idx> decode_class(const Tab<Idx>& T, const cell::Pair<Idx> (*ct)[ce
     k.sr = r;
     k.word = word << (2 * p);
     k.h = h;
+    return k;
+}
+
+// Decode class number c among the classes of (p, d) whose P' and S' stay at heights
+// <= the cap of ct: P' as above with capped counts, then S' by its capped counts
+// (rows 0..p-3 of ct) while its rank is summed with the full table, so the class is
+// what decode_class gives for its own number.
+template <typename Idx>
+OFP_HD Class<Idx> decode_class_capped(const Tab<Idx>& T, const cell::Pair<Idx> (*ct)[cell::LdsCols<Idx>::value], int W,
+                                      int p, int d, uint64_t c) {
+    Class<Idx> k = decode_class<Idx>(T, ct, W, p, c);
+    Idx r = k.sr, sr = 0;
+    int h = k.h + d;
+    for (int pos = p - 3; pos >= 0; --pos) {
+        const cell::Pair<Idx> g = ct[pos][h];
+        const Z2<Idx> e = ldz(T.q[pos][h]);
+        const bool g0 = r >= g.n, g1 = r >= g.c;
+        r -= g1 ? g.c : (g0 ? g.n : Idx(0));
+        sr += g1 ? e.zc : (g0 ? e.zn : Idx(0));
+        h += g1 ? 1 : (g0 ? -1 : 0);
+    }
+    k.sr = sr;
     return k;
 }
 
@@ -518,20 +541,20 @@ OFP_HD void pair_body(const PairLaunch& a, const Tab<Idx>& T, const Class<Idx>& 
     }
 }
 
-// Class completion table of (p, d) from the plain height table d0
-// (kDpRows x kDpCols): out[m][h] = {G[m-1][h], G[m-1][h] + G[m-1][h-1]} for
-// m in p+1..kDpRows-1 (other rows zero).  Returns G[W-1][1] for W = kDpRows-1
-// unused; the class count of an n-row is g[W-1][1], see class_count().
-inline void build_class_table(const uint64_t (*d0)[kDpCols], int p, int d, uint64_t (*g)[kDpCols]) {
+// Class completion table of (p, d) from a height table d0 (kDpRows x kDpCols; plain,
+// or capped at cap): g[m][h] = G_d[m][h] for m >= p, other rows zero.  cap > 0: the
+// classes whose P' and S' stay at heights <= cap.
+inline void build_class_table(const uint64_t (*d0)[kDpCols], int p, int d, uint64_t (*g)[kDpCols], int cap = 0) {
+    const int top = cap > 0 ? cap : kDpCols - 1;  // the greatest height counted
     for (int m = 0; m < kDpRows; ++m)
         for (int h = 0; h < kDpCols; ++h) g[m][h] = 0;
-    for (int h = 0; h < kDpCols; ++h) {
+    for (int h = 0; h <= top; ++h) {
         const int e = h + d;
-        g[p][h] = (p >= 2 && e >= 0 && e < kDpCols) ? d0[p - 2][e] : 0;
+        g[p][h] = (p >= 2 && e >= 0 && e <= top) ? d0[p - 2][e] : 0;
     }
     for (int m = p + 1; m < kDpRows; ++m)
-        for (int h = 0; h < kDpCols; ++h)
-            g[m][h] = g[m - 1][h] + (h > 0 ? g[m - 1][h - 1] : 0) + (h + 1 < kDpCols ? g[m - 1][h + 1] : 0);
+        for (int h = 0; h <= top; ++h)
+            g[m][h] = g[m - 1][h] + (h > 0 ? g[m - 1][h - 1] : 0) + (h + 1 <= top ? g[m - 1][h + 1] : 0);
 }
 
 }  // namespace pair
@@ -541,27 +564,26 @@ namespace ofp {
 namespace pair {
 
 // Packed class table of (p, d) with C columns per row: row m holds
-// {G_d[m-1][h], G_d[m-1][h] + G_d[m-1][h-1]} for m > p (rows <= p are zero);
-// C = cell::LdsCols<Idx>::value, the layout the kernels keep in LDS.
+// {G_d[m-1][h], G_d[m-1][h] + G_d[m-1][h-1]} for m > p; with a cap (d0: the height
+// table capped there) rows m <= p - 3 hold the capped height table's entries, which
+// count S'; other rows are zero.  C = cell::LdsCols<Idx>::value, the layout the
+// kernels keep in LDS.
 template <typename Idx, int C>
-inline void pack_class_table(const uint64_t (*d0)[kDpCols], int p, int d, cell::Pair<Idx> (*out)[C]) {
+inline void pack_class_table(const uint64_t (*d0)[kDpCols], int p, int d, cell::Pair<Idx> (*out)[C], int cap = 0) {
     uint64_t g[kDpRows][kDpCols];
-    build_class_table(d0, p, d, g);
+    build_class_table(d0, p, d, g, cap);
     for (int m = 0; m < kDpRows; ++m)
         for (int h = 0; h < C; ++h) {
-            out[m][h].n = 0;
-            out[m][h].c = 0;
-            if (m > p && m >= 1) {
-                out[m][h].n = (Idx)g[m - 1][h];
-                out[m][h].c = (Idx)(g[m - 1][h] + (h > 0 ? g[m - 1][h - 1] : 0));
-            }
+            const uint64_t* row = m > p && m >= 1 ? g[m - 1] : (cap > 0 && m <= p - 3 ? d0[m] : nullptr);
+            out[m][h].n = row ? (Idx)row[h] : Idx(0);
+            out[m][h].c = row ? (Idx)(row[h] + (h > 0 ? row[h - 1] : 0)) : Idx(0);
         }
 }
 
 // Classes of (p, d) in an n-row: G_d[W-1][1].
-inline uint64_t class_count(const uint64_t (*d0)[kDpCols], int W, int p, int d) {
+inline uint64_t class_count(const uint64_t (*d0)[kDpCols], int W, int p, int d, int cap = 0) {
     uint64_t g[kDpRows][kDpCols];
-    build_class_table(d0, p, d, g);
+    build_class_table(d0, p, d, g, cap);
     return W - 1 >= p ? g[W - 1][1] : 0;
 }
 
