@@ -48,7 +48,7 @@ struct Sweep {
     bool fixed = false;        // buffers are slices of the library's static device array (no graphs)
     int row = -1;              // rows swept since the initial state; -1: state of unknown origin
     std::vector<hipEvent_t> seg_ev;  // timing events of row segments (ofp_row_sweep)
-    uint64_t* acc = nullptr;         // the k sums of a half-row solve's last step (zeroed with the state)
+    uint64_t* acc = nullptr;         // the sums of a half-row solve's last step (zeroed with the state)
     uint32_t* gscratch = nullptr;    // its scratch (states of more than 20 positions)
     size_t gscratch_cap = 0;
     // pair passes: two more streams for the launches of one pass that may run
@@ -348,7 +348,7 @@ ofp_status ensure_state(ofp_ctx* c, Sweep& s, int n, const uint32_t* moduli, int
         s.mods_cap = 0;
         const int cap = std::max(k, 16);
         OFP_HIP(c, sweep_alloc(s, (void**)&s.mods_dev, cap * sizeof(uint32_t)), "allocate moduli");
-        OFP_HIP(c, sweep_alloc(s, (void**)&s.acc, cap * sizeof(uint64_t)), "allocate sums");
+        OFP_HIP(c, sweep_alloc(s, (void**)&s.acc, cap * sizeof(uint64_t) * glue::kAccWords), "allocate sums");
         s.mods_cap = cap;
     }
     s.mods.assign(moduli, moduli + k);
@@ -866,8 +866,9 @@ ofp_status init_state(ofp_ctx* c, Sweep& s) {
     s.row = 0;
     uint64_t start = dp_at(s.W - 1, 1);
     hipError_t e = s.mods_dev
-                       ? launch_set_one(s.main, start, s.Kp, s.K, s.layout, s.mods_dev, s.acc, s.stream)
-                       : launch_set_one_values(s.main, start, s.Kp, s.K, s.layout, s.mods.data(), s.acc, s.stream);
+                       ? launch_set_one(s.main, start, s.Kp, s.K, s.layout, s.mods_dev, s.acc, glue::kAccWords * s.K, s.stream)
+                       : launch_set_one_values(s.main, start, s.Kp, s.K, s.layout, s.mods.data(), s.acc, glue::kAccWords * s.K,
+                                               s.stream);
     if (e != hipSuccess) return hip_fail(c, e, "init kernel");
     return OFP_OK;
 }
@@ -1053,7 +1054,7 @@ ofp_status ofp_create(const ofp_config* cfg, ofp_ctx** out) {
         for (int q = 0; q < 32; ++q)
             c->binom[p * 32 + q] = q == 0 ? 1 : (p == 0 ? 0 : c->binom[(p - 1) * 32 + q] + c->binom[(p - 1) * 32 + q - 1]);
     const size_t bal = (sizeof(glue::Ballot) + 255) / 256 * 256, bin = (sizeof c->binom + 255) / 256 * 256;
-    if (bad(hipMalloc(&c->gdev, bal + bin + kMaxKC * sizeof(uint64_t)))) return OFP_E_RUNTIME;
+    if (bad(hipMalloc(&c->gdev, bal + bin + kMaxKC * sizeof(uint64_t) * glue::kAccWords))) return OFP_E_RUNTIME;
     c->dballot = reinterpret_cast<const glue::Ballot*>(c->gdev);
     c->dbinom = reinterpret_cast<const uint32_t*>(c->gdev + bal);
     c->static_acc = reinterpret_cast<uint64_t*>(c->gdev + bal + bin);

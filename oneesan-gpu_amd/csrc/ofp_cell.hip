@@ -193,10 +193,11 @@ __global__ void fill_remote_kernel(uint32_t* main, uint64_t m0, uint64_t M, uint
 }
 
 __global__ void set_one_kernel(uint32_t* main, uint64_t index, int K, int k, int layout,
-                               const uint32_t* mods, uint64_t* acc) {
+                               const uint32_t* mods, uint64_t* acc, int accs) {
     int j = threadIdx.x;
     if (j < k) main[state_elem(layout, index, K, j)] = 1u % mods[j];
-    if (j < k && acc) acc[j] = 0;
+    if (acc)
+        for (int i = j; i < accs; i += blockDim.x) acc[i] = 0;
 }
 
 template <typename Idx, int KC>
@@ -315,26 +316,28 @@ struct ModVals {
     uint32_t m[kMaxKC];
 };
 __global__ void set_one_values_kernel(uint32_t* main, uint64_t index, int K, int k, int layout, ModVals mods,
-                                      uint64_t* acc) {
+                                      uint64_t* acc, int accs) {
     int j = threadIdx.x;
     if (j < k) main[state_elem(layout, index, K, j)] = 1u % mods.m[j];
-    if (j < k && acc) acc[j] = 0;
+    if (acc)
+        for (int i = j; i < accs; i += blockDim.x) acc[i] = 0;
 }
 
 hipError_t launch_set_one_values(uint32_t* main, uint64_t index, int K, int k, int layout,
-                                 const uint32_t* mods_host, uint64_t* acc, hipStream_t s) {
+                                 const uint32_t* mods_host, uint64_t* acc, int accs,
+                                 hipStream_t s) {
     if (k < 1 || k > kMaxKC || K < k) return hipErrorInvalidValue;
     ModVals mv{};
     for (int j = 0; j < k; ++j) mv.m[j] = mods_host[j];
-    hipLaunchKernelGGL(set_one_values_kernel, dim3(1), dim3(64), 0, s, main, index, K, k, layout, mv, acc);
+    hipLaunchKernelGGL(set_one_values_kernel, dim3(1), dim3(64), 0, s, main, index, K, k, layout, mv, acc, accs);
     return hipGetLastError();
 }
 
 hipError_t launch_set_one(uint32_t* main, uint64_t index, int K, int k, int layout,
-                          const uint32_t* mods_dev, uint64_t* acc, hipStream_t s) {
+                          const uint32_t* mods_dev, uint64_t* acc, int accs, hipStream_t s) {
     if (k < 1 || k > 1024 || K < k) return hipErrorInvalidValue;
     hipLaunchKernelGGL(set_one_kernel, dim3(1), dim3(((k + 63) / 64) * 64), 0, s, main, index, K, k,
-                       layout, mods_dev, acc);
+                       layout, mods_dev, acc, accs);
     return hipGetLastError();
 }
 

@@ -24,19 +24,23 @@ struct Tables {
 };
 constexpr int kTableSets = 2;  // up to kBaseStrands, and m = 19
 
+// Accumulators of a sum: eight sets (one per XCD's workgroups) of three 64-bit parts.
+constexpr int kCopies = 8;
+constexpr int kAccWords = 3 * kCopies;
+
 struct GlueLaunch {
     const uint32_t* main;   // the frontier after half of the cells, state-major, stride K
     const uint32_t* blk;
     const void* dp;         // packed height table (cell::Quad)
     const Ballot* ballot;
     const uint32_t* binom;  // C(p, q) at p * 32 + q
-    uint64_t* acc;          // k sums, zero before the first launch
+    uint64_t* acc;          // kAccWords sums per modulus, zero before the first launch
     const uint32_t* mods;   // k moduli on the device, or null: mod
     uint32_t* scratch;      // lower words of a batch (more than kTabStrands strands)
     int W, K, k;
     int center;             // the cut vertex of an odd row, -1 for even W
     int segs;
-    uint32_t tasks, ystride, task0, batch;
+    uint32_t tasks, piece, ystride, task0, batch;
     uint32_t from, to, each;  // scratch entries of a task: of the level read, of the one written, in all
     int removed;              // arcs removed at the level read
     Seg seg[6];

@@ -11,8 +11,8 @@
 //  * Lists: rows sorted by length, slices of 64 rows (one wave), 8 columns of 16
 //    bits per lane and chunk, so a wave reads its lists as whole 1 KB chunks.
 //    Shorter rows are filled up with column B, a zero entry.
-//  * LDS: KC moduli per pass (grid.y walks the moduli), KC chosen so that the B
-//    entries fit: 4 up to m = 17 (78 KB), 2 at m = 19 (134 KB of the 160).  A team
+//  * LDS: KC moduli per pass, KC chosen so that the B entries fit: 4 up to m = 17
+//    (78 KB), 2 at m = 19 (134 of the 160 KB).  A team
 //    of waves shares one task: one wave up to m = 11 (132 rows), a workgroup of 4
 //    waves for m = 13 and 15, of 16 above.
 //  * m = 21 (58786 words, 235 KB at one modulus) and 23: the lower words are
@@ -40,14 +40,12 @@ __device__ __forceinline__ void load_rec(const uint32_t* base, uint64_t i, int K
     if constexpr (KC == 1) {
         v[0] = q[0];
     } else {
-        const uint2 a = *reinterpret_cast<const uint2*>(q);
-        v[0] = a.x;
-        v[1] = a.y;
-        if constexpr (KC == 4) {
-            uint2 b = make_uint2(0u, 0u);
-            if (off + 2 < K) b = *reinterpret_cast<const uint2*>(q + 2);
-            v[2] = b.x;
-            v[3] = b.y;
+#pragma unroll
+        for (int j = 0; j < KC; j += 2) {
+            uint2 t = make_uint2(0u, 0u);
+            if (j == 0 || off + j < K) t = *reinterpret_cast<const uint2*>(q + j);
+            v[j] = t.x;
+            v[j + 1] = t.y;
         }
     }
 }
@@ -88,15 +86,38 @@ struct Sum {
             hi[j] += (p >> 32) + (uint64_t)x[j] * (uint32_t)(acc[j] >> 32);
         }
     }
-    // The wave's sum mod each modulus into the accumulators (64-bit adds of values below 2^32).
-    __device__ void flush(const GlueLaunch& a, int off, const uint32_t (&mod)[KC]) const {
+    // The workgroup's sums (of moduli off..) into one of the kCopies sets of
+    // accumulators: per modulus the low sums, and the high sums in two halves (a
+    // workgroup's stay below 2^63: a lane adds at most 2^13 products of a residue and
+    // a sum below 2^43), reduced by the last kernel.
+    template <int NT>
+    __device__ void flush(const GlueLaunch& a, int off) {
+        __shared__ unsigned long long part[NT / 64][2 * KC];
+        const int wave = (int)threadIdx.x >> 6;
 #pragma unroll
         for (int j = 0; j < KC; ++j) {
-            const uint64_t m = mod[j];
-            uint32_t r = (uint32_t)((lo[j] % m + (hi[j] % m) * ((1ull << 32) % m)) % m);
-            for (int d = 32; d >= 1; d >>= 1) r = addm(r, (uint32_t)__shfl_xor((int)r, d), mod[j]);
-            if ((threadIdx.x & 63) == 0 && off + j < a.k)
-                atomicAdd(reinterpret_cast<unsigned long long*>(a.acc) + off + j, (unsigned long long)r);
+            for (int d = 32; d >= 1; d >>= 1) {
+                lo[j] += __shfl_xor((unsigned long long)lo[j], d);
+                hi[j] += __shfl_xor((unsigned long long)hi[j], d);
+            }
+            if ((threadIdx.x & 63) == 0) {
+                part[wave][j] = lo[j];
+                part[wave][KC + j] = hi[j];
+            }
+        }
+        __syncthreads();
+        const int j = (int)threadIdx.x;
+        if (j < KC && off + j < a.k) {
+            unsigned long long l = 0, h = 0;
+            for (int w = 0; w < NT / 64; ++w) {
+                l += part[w][j];
+                h += part[w][KC + j];
+            }
+            unsigned long long* acc =
+                reinterpret_cast<unsigned long long*>(a.acc) + (size_t)(blockIdx.x & (kCopies - 1)) * 3 * a.k + off + j;
+            atomicAdd(acc, l);
+            atomicAdd(acc + a.k, h & 0xffffffffull);
+            atomicAdd(acc + 2 * a.k, h >> 32);
         }
     }
 };
@@ -129,9 +150,11 @@ __device__ __forceinline__ void add_lists(const Seg& g, uint32_t slice, const Y&
     for (int j = 0; j < KC; ++j) acc[j] = 0;
     const uint32_t c1 = g.sptr[slice + 1];
     const uint4* cols = g.cols + (size_t)(threadIdx.x & 63);
-    for (uint32_t c = g.sptr[slice]; c < c1; ++c) {
-        const uint4 q = cols[(size_t)c * 64];
-        const uint32_t w[4] = {q.x, q.y, q.z, q.w};
+    uint32_t c = g.sptr[slice];
+    uint4 next = cols[(size_t)c * 64];  // the next chunk is loaded while one is added
+    for (; c < c1; ++c) {
+        const uint32_t w[4] = {next.x, next.y, next.z, next.w};
+        if (c + 1 < c1) next = cols[(size_t)(c + 1) * 64];
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             const Entry<KC> e0 = y(w[i] & 0xffffu), e1 = y(w[i] >> 16);
@@ -141,28 +164,43 @@ __device__ __forceinline__ void add_lists(const Seg& g, uint32_t slice, const Y&
     }
 }
 
-// Tasks in LDS: teams of TW waves, one occupancy per team at a time.
+// Tasks in LDS: teams of TW waves, one occupancy per team at a time.  The words of
+// one occupancy lie scattered, but next to those of the occupancies that differ in
+// the lowest positions -- the tasks with the next numbers -- and a record's moduli
+// are read by different passes.  So block b works on XCD b % 8 (round-robin
+// dispatch), the passes of a task are neighbouring blocks of one XCD, and the tasks
+// go to the XCDs in pieces of a.piece per team (32, fewer where an XCD would get less
+// than eight pieces): what one fetches from HBM the others find in that XCD's L2.
 template <int KC, typename Idx, int NT, int TW>
 __global__ __launch_bounds__(NT) void glue_kernel(GlueLaunch a) {
     constexpr int kTeams = NT / 64 / TW;
     extern __shared__ __align__(16) unsigned char lds[];
     __shared__ Pair<Idx> D[kMaxW][kCols];
+    __shared__ uint32_t binom[kMaxW * 32];
     load_height<Idx>(D, a.dp);
+    for (int t = threadIdx.x; t < a.W * 32; t += NT) binom[t] = a.binom[t];
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const int team = wave / TW, tlane = (int)threadIdx.x - team * TW * 64;
     Entry<KC>* y = reinterpret_cast<Entry<KC>*>(lds + (size_t)team * a.ystride);
-    const int off = (int)blockIdx.y * KC;
+    const uint32_t xcd = blockIdx.x & 7u, local = blockIdx.x >> 3, passes = (uint32_t)(a.K + KC - 1) / KC;
+    const uint32_t nw = (gridDim.x >> 3) / passes;  // blocks of one pass on one XCD
+    const int off = (int)(local % passes) * KC;
     uint32_t mod[KC];
     load_mods<KC>(a, off, mod);
     Sum<KC> sum;
     sum.init();
     __syncthreads();
-    for (uint32_t t = blockIdx.x * kTeams + team; t < a.tasks; t += gridDim.x * kTeams) {
+    const uint32_t P = a.piece * kTeams;
+    for (uint32_t q = local / passes * kTeams;; q += nw * kTeams) {
+        const uint32_t first = (q / P * 8 + xcd) * P + q % P;
+        if (first >= a.tasks) break;  // later rounds lie higher
+        const uint32_t t = first + (uint32_t)team;
+        if (t >= a.tasks) continue;   // (one-wave teams only: no barrier in their rounds)
         int gi = 0;
         uint32_t idx = t;
         while (idx >= a.seg[gi].count) idx -= a.seg[gi++].count;
         const Seg& g = a.seg[gi];
-        const uint32_t occ = mask_of(a.binom, a.W, g.m, idx);
+        const uint32_t occ = __builtin_amdgcn_readfirstlane((int)mask_of(binom, a.W, g.m, idx));
         const int weight = mask_weight(occ, a.W, a.center);
         if (!weight) continue;
         const uint32_t rocc = reversed_mask(occ, a.W);
@@ -185,7 +223,7 @@ __global__ __launch_bounds__(NT) void glue_kernel(GlueLaunch a) {
         if constexpr (TW > 1) __syncthreads();
         else __threadfence_block();
     }
-    sum.flush(a, off, mod);
+    sum.template flush<NT>(a, off);
 }
 
 // ---- strands beyond the lists ----
@@ -319,15 +357,21 @@ __global__ __launch_bounds__(256) void glue_big_kernel(GlueLaunch a) {
         }
         sum.add(x, acc);
     }
-    sum.flush(a, off, mod);
+    sum.template flush<256>(a, off);
 }
 
-// The answer word (index 0) takes the sums.
-__global__ void glue_finish_kernel(GlueLaunch a, uint32_t* main) {
-    for (int j = threadIdx.x; j < a.k; j += blockDim.x) {
-        const uint32_t m = a.mods ? a.mods[j] : a.mod[j];
-        main[j] = (uint32_t)(a.acc[j] % m);
-    }
+// The answer word (index 0) takes the sums, one wave per modulus: low + 2^32 (mid +
+// 2^32 high), each below 2^63 over all waves.
+__global__ __launch_bounds__(64) void glue_finish_kernel(GlueLaunch a, uint32_t* main) {
+    const int j = (int)blockIdx.x, lane = (int)threadIdx.x;
+    const uint64_t m = a.mods ? a.mods[j] : a.mod[j];
+    uint64_t v = lane < kAccWords ? a.acc[(size_t)lane * a.k + j] % m : 0;  // lane = copy * 3 + part
+    const uint64_t two32 = (1ull << 32) % m;
+    const int part = lane % 3;
+    if (part >= 1) v = v * two32 % m;
+    if (part == 2) v = v * two32 % m;
+    for (int d = 32; d >= 1; d >>= 1) v += __shfl_xor((unsigned long long)v, d);
+    if (lane == 0) main[j] = (uint32_t)(v % m);
 }
 
 // ---- lists, m strands from m - 2 ----
@@ -514,7 +558,8 @@ hipError_t launch_lds(const GlueLaunch& a, uint32_t blocks, hipStream_t s) {
                                                  (int)bytes);
         if (e != hipSuccess) return e;
     }
-    hipLaunchKernelGGL(k, dim3(blocks, (a.K + KC - 1) / KC), dim3(NT), bytes, s, a);
+    const uint32_t passes = (uint32_t)(a.K + KC - 1) / KC;  // blocks: whole rounds of 8 XCDs and all passes
+    hipLaunchKernelGGL(k, dim3(std::max(1u, blocks / (8 * passes)) * 8 * passes), dim3(NT), bytes, s, a);
     return hipGetLastError();
 }
 
@@ -603,13 +648,16 @@ hipError_t launch_idx(GlueLaunch a, const Tables* tabs, const Ballot& hb, const 
             a.tasks += a.seg[a.segs++].count;
         }
         if (!a.tasks) continue;
+        a.piece = std::min(32u, std::max(1u, a.tasks / (64u * (c.hi <= 11 ? 4u : 1u))));
+        // resident workgroups (the LDS and registers of a class), fewer where a team
+        // would get less than two tasks per pass
         const uint32_t cu = (uint32_t)cus;
-        if (c.lo >= 17)
-            e = launch_lds_kc<Idx, 1024, 16>(a, c.lo == 19 ? 2 : 4, std::min(a.tasks, cu * (c.lo == 19 ? 1 : 2)), s);
-        else if (c.lo >= 13)
-            e = launch_lds_kc<Idx, 256, 4>(a, 4, std::min(a.tasks, cu * 8), s);
-        else
-            e = launch_lds_kc<Idx, 256, 1>(a, 4, std::min((a.tasks + 3) / 4, cu * 8), s);
+        const auto blocks = [&](uint32_t most, uint32_t teams) {
+            return std::min(most, std::max(cu, (a.tasks + 2 * teams - 1) / (2 * teams) * (uint32_t)((a.K + 3) / 4)));
+        };
+        if (c.lo >= 17) e = launch_lds_kc<Idx, 1024, 16>(a, c.lo == 19 ? 2 : 4, blocks(cu * 2, 1), s);
+        else if (c.lo >= 13) e = launch_lds_kc<Idx, 256, 4>(a, 4, blocks(cu * 8, 1), s);
+        else e = launch_lds_kc<Idx, 256, 1>(a, 4, blocks(cu * 8, 4), s);
         if (launches) ++*launches;
     }
     return e;
@@ -628,7 +676,7 @@ hipError_t launch_glue(const GlueLaunch& a, const Tables* tabs, const Ballot& hb
     const hipError_t e = wide ? launch_idx<uint64_t>(a, tabs, hb, binom, cus, scratch_bytes, s, launches)
                               : launch_idx<uint32_t>(a, tabs, hb, binom, cus, scratch_bytes, s, launches);
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(glue_finish_kernel, dim3(1), dim3(64), 0, s, a, main_out);
+    hipLaunchKernelGGL(glue_finish_kernel, dim3(a.k), dim3(64), 0, s, a, main_out);
     if (launches) ++*launches;
     return hipGetLastError();
 }

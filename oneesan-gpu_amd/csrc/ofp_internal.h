@@ -89,12 +89,13 @@ hipError_t launch_fill_remote(uint32_t* main, uint64_t m0, uint64_t M, uint32_t*
                               uint64_t B, int K, int k, const uint32_t* mods_dev, uint64_t seed,
                               hipStream_t s);
 // Set main[(index, j)] = 1 mod moduli[j] for j < k (interleave stride K) and, where
-// acc is given, its k sums to zero.
+// acc is given, its accs sums to zero.
 hipError_t launch_set_one(uint32_t* main, uint64_t index, int K, int k, int layout,
-                          const uint32_t* mods_dev, uint64_t* acc, hipStream_t s);
+                          const uint32_t* mods_dev, uint64_t* acc, int accs, hipStream_t s);
 // The same with the moduli passed by value from host memory (k <= kMaxKC).
 hipError_t launch_set_one_values(uint32_t* main, uint64_t index, int K, int k, int layout,
-                                 const uint32_t* mods_host, uint64_t* acc, hipStream_t s);
+                                 const uint32_t* mods_host, uint64_t* acc, int accs,
+                                 hipStream_t s);
 
 // ---- pair pass (ofp_pair.hip; launch struct pair::PairLaunch in ofp_pair_impl.h) ----
 namespace pair { struct PairLaunch; }
