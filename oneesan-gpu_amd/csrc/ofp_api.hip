@@ -104,6 +104,8 @@ struct ofp_ctx {
         char* tables = nullptr;
         std::vector<uint64_t> mc, bc;  // words per group
     } last_low;
+    uint32_t* io = nullptr;  // stride changes between callers' arrays and the device
+    size_t io_bytes = 0;
     char* stage = nullptr;  // exchange buffer: plan tables and staging buckets, reused
     size_t stage_bytes = 0;
     // half-row solves (ofp_glue_impl.h): the ballot and binomial tables (host copies
@@ -892,6 +894,63 @@ int moduli_groups(int k, int g, int* sizes, int cap) {
     return i;
 }
 
+// Residues between a caller's state-major array (n states of k) and device words in a
+// layout with stride Kp.  Equal strides (k = 1 or even, state-major) copy at once;
+// others go through a device buffer of at most kIoBytes, where a kernel changes the
+// stride, so the host never touches single residues.
+constexpr size_t kIoBytes = 64ull << 20;
+ofp_status io_buffer(ofp_ctx* c, size_t bytes, uint32_t** out) {
+    bytes = std::min(bytes, kIoBytes);
+    if (c->io_bytes < bytes) {
+        if (c->io) OFP_HIP(c, hipFree(c->io), "free copy buffer");
+        c->io = nullptr;
+        c->io_bytes = 0;
+        OFP_HIP(c, hipMalloc(&c->io, bytes), "copy buffer");
+        c->io_bytes = bytes;
+    }
+    *out = c->io;
+    return OFP_OK;
+}
+// States per piece: a multiple of the 64 states of a tile.
+uint64_t io_piece(const ofp_ctx* c, int k) { return std::max<uint64_t>(c->io_bytes / ((size_t)k * 4) / 64 * 64, 64); }
+
+ofp_status upload_states(ofp_ctx* c, uint32_t* dev, const uint32_t* host, uint64_t n, int k, int Kp, int layout,
+                         hipStream_t s, const char* what) {
+    if (!n) return OFP_OK;
+    if (layout == 1 && Kp == k) {
+        OFP_HIP(c, hipMemcpy(dev, host, n * (size_t)k * 4, hipMemcpyHostToDevice), what);
+        return OFP_OK;
+    }
+    uint32_t* io = nullptr;
+    if (ofp_status st = io_buffer(c, std::max<uint64_t>(n, 64) * k * 4, &io)) return st;
+    const uint64_t piece = io_piece(c, k);
+    for (uint64_t i = 0; i < n; i += piece) {
+        const uint64_t m = std::min(piece, n - i);
+        OFP_HIP(c, hipMemcpy(io, host + i * k, m * (size_t)k * 4, hipMemcpyHostToDevice), what);
+        OFP_HIP(c, launch_restride(dev, io, i, m, k, Kp, layout, true, s), what);
+        OFP_HIP(c, hipStreamSynchronize(s), what);
+    }
+    return OFP_OK;
+}
+ofp_status download_states(ofp_ctx* c, uint32_t* host, uint32_t* dev, uint64_t n, int k, int Kp, int layout, hipStream_t s,
+                           const char* what) {
+    if (!n) return OFP_OK;
+    if (layout == 1 && Kp == k) {
+        OFP_HIP(c, hipMemcpy(host, dev, n * (size_t)k * 4, hipMemcpyDeviceToHost), what);
+        return OFP_OK;
+    }
+    uint32_t* io = nullptr;
+    if (ofp_status st = io_buffer(c, std::max<uint64_t>(n, 64) * k * 4, &io)) return st;
+    const uint64_t piece = io_piece(c, k);
+    for (uint64_t i = 0; i < n; i += piece) {
+        const uint64_t m = std::min(piece, n - i);
+        OFP_HIP(c, launch_restride(dev, io, i, m, k, Kp, layout, false, s), what);
+        OFP_HIP(c, hipStreamSynchronize(s), what);
+        OFP_HIP(c, hipMemcpy(host + i * k, io, m * (size_t)k * 4, hipMemcpyDeviceToHost), what);
+    }
+    return OFP_OK;
+}
+
 // Host rank / unrank over the height table (lexicographic, N<R<L, entered at height 1).
 uint64_t rank_word(uint64_t w, int width) {
     uint64_t r = 0;
@@ -1390,28 +1449,22 @@ ofp_status ofp_apply_cells(ofp_ctx* c, int n, const uint32_t* moduli, int k, uin
     ofp_status s = ensure_state(c, sw, n, moduli, k);
     const bool pairs = pairs_apply(c, n) && p_hi - p_lo >= 1;
     if (s) return s;
-    // host state-major (index*k + j) <-> device layout
-    const int Kp = sw.Kp, lay = sw.layout;
-    std::vector<uint32_t> tm(padded_states(sw.nmain) * (size_t)Kp, 0),
-        tb(padded_states(sw.nblk ? sw.nblk : 1) * (size_t)Kp, 0);
-    for (uint64_t i = 0; i < sw.nmain; ++i)
-        for (int j = 0; j < k; ++j) tm[state_elem(lay, i, Kp, j)] = main_io[i * k + j];
-    for (uint64_t i = 0; i < sw.nblk; ++i)
-        for (int j = 0; j < k; ++j) tb[state_elem(lay, i, Kp, j)] = blocked_io[i * k + j];
-    OFP_HIP(c, hipMemcpy(sw.main, tm.data(), tm.size() * 4, hipMemcpyHostToDevice), "upload main");
-    OFP_HIP(c, hipMemcpy(sw.blk, tb.data(), tb.size() * 4, hipMemcpyHostToDevice), "upload blocked");
+    s = upload_states(c, sw.main, main_io, sw.nmain, k, sw.Kp, sw.layout, sw.stream, "upload main");
+    if (s) return s;
+    if (blocked_valid) {  // else the first cell reads none and writes all (cell 1: none)
+        s = upload_states(c, sw.blk, blocked_io, sw.nblk, k, sw.Kp, sw.layout, sw.stream, "upload blocked");
+        if (s) return s;
+    }
     sw.row = -1;  // arbitrary state: no height caps
     s = pairs ? enqueue_pairs(c, sw, p_hi, p_lo, blocked_valid != 0, nullptr)
               : enqueue_cells(c, sw, p_hi, p_lo, blocked_valid != 0, nullptr);
     if (s) return s;
     OFP_HIP(c, hipStreamSynchronize(sw.stream), "apply sync");
-    OFP_HIP(c, hipMemcpy(tm.data(), sw.main, tm.size() * 4, hipMemcpyDeviceToHost), "download main");
-    OFP_HIP(c, hipMemcpy(tb.data(), sw.blk, tb.size() * 4, hipMemcpyDeviceToHost), "download blocked");
-    for (uint64_t i = 0; i < sw.nmain; ++i)
-        for (int j = 0; j < k; ++j) main_io[i * k + j] = tm[state_elem(lay, i, Kp, j)];
+    s = download_states(c, main_io, sw.main, sw.nmain, k, sw.Kp, sw.layout, sw.stream, "download main");
+    if (s) return s;
+    if (p_lo > 1) return download_states(c, blocked_io, sw.blk, sw.nblk, k, sw.Kp, sw.layout, sw.stream, "download blocked");
     // after cell 1 nothing is blocked; the device buffer is simply not written
-    for (uint64_t i = 0; i < sw.nblk; ++i)
-        for (int j = 0; j < k; ++j) blocked_io[i * k + j] = (p_lo == 1) ? 0u : tb[state_elem(lay, i, Kp, j)];
+    std::memset(blocked_io, 0, sw.nblk * (size_t)k * 4);
     return OFP_OK;
 }
 
@@ -1516,18 +1569,11 @@ ofp_status ofp_shard_sweep(ofp_ctx* c, const ofp_shard_spec* sp, ofp_shard_info*
     unsigned long long stray = 0;
     OFP_HIP_R(hipMemcpy(&stray, dstray, sizeof stray, hipMemcpyDeviceToHost), "read counter");
     info->stray_stores = stray;
-    if (main_out || blk_out) {
-        std::vector<uint32_t> t(std::max(M, B) * (size_t)Kp);
-        if (main_out && M) {
-            OFP_HIP_R(hipMemcpy(t.data(), dm, M * Kp * 4, hipMemcpyDeviceToHost), "download main");
-            for (uint64_t i = 0; i < M; ++i)
-                for (int j = 0; j < k; ++j) main_out[i * k + j] = t[i * Kp + j];
-        }
-        if (blk_out && B) {
-            OFP_HIP_R(hipMemcpy(t.data(), db, B * Kp * 4, hipMemcpyDeviceToHost), "download blocked");
-            for (uint64_t i = 0; i < B; ++i)
-                for (int j = 0; j < k; ++j) blk_out[i * k + j] = t[i * Kp + j];
-        }
+    if (main_out) st = download_states(c, main_out, dm, M, k, Kp, 1, c->stream, "download main");
+    if (!st && blk_out) st = download_states(c, blk_out, db, B, k, Kp, 1, c->stream, "download blocked");
+    if (st) {
+        release();
+        return st;
     }
 #undef OFP_HIP_R
     release();
@@ -1686,19 +1732,11 @@ ofp_status ofp_group_sweep(ofp_ctx* c, const ofp_group_spec* sp, ofp_group_info*
         if (ctbytes) OFP_HIP_R(hipMemcpy(dct, cts.data(), ctbytes, hipMemcpyHostToDevice), "upload class tables");
     }
     OFP_HIP_R(hipMemcpy(dmods, sp->moduli, k * 4, hipMemcpyHostToDevice), "copy moduli");
-    const bool blk_in = sp->high && blk_io;
-    if (main_io || blk_in) {
-        std::vector<uint32_t> t(std::max<uint64_t>(std::max(M, B), 1) * Kp, 0);
-        if (main_io) {
-            for (uint64_t i = 0; i < M; ++i)
-                for (int j = 0; j < k; ++j) t[i * Kp + j] = main_io[i * k + j];
-            OFP_HIP_R(hipMemcpy(dm, t.data(), M * Kp * 4, hipMemcpyHostToDevice), "upload main window");
-        }
-        if (blk_in) {
-            for (uint64_t i = 0; i < B; ++i)
-                for (int j = 0; j < k; ++j) t[i * Kp + j] = blk_io[i * k + j];
-            OFP_HIP_R(hipMemcpy(db, t.data(), B * Kp * 4, hipMemcpyHostToDevice), "upload blocked window");
-        }
+    if (main_io) st = upload_states(c, dm, main_io, M, k, Kp, 1, c->stream, "upload main window");
+    if (!st && sp->high && blk_io) st = upload_states(c, db, blk_io, B, k, Kp, 1, c->stream, "upload blocked window");
+    if (st) {
+        release();
+        return st;
     }
     // Seeded inputs, one hash domain per window start and half: main words
     // unless given, blocked words only where the first cell reads them.
@@ -1848,19 +1886,11 @@ ofp_status ofp_group_sweep(ofp_ctx* c, const ofp_group_spec* sp, ofp_group_info*
         lw.bc = bc;
         lw.valid = true;
     }
-    const bool blk_out = !sp->high && blk_io;
-    if (main_io || blk_out) {
-        std::vector<uint32_t> t(std::max<uint64_t>(std::max(M, B), 1) * Kp);
-        if (main_io && M) {
-            OFP_HIP_R(hipMemcpy(t.data(), dm, M * Kp * 4, hipMemcpyDeviceToHost), "download main window");
-            for (uint64_t i = 0; i < M; ++i)
-                for (int j = 0; j < k; ++j) main_io[i * k + j] = t[i * Kp + j];
-        }
-        if (blk_out && B) {
-            OFP_HIP_R(hipMemcpy(t.data(), db, B * Kp * 4, hipMemcpyDeviceToHost), "download blocked window");
-            for (uint64_t i = 0; i < B; ++i)
-                for (int j = 0; j < k; ++j) blk_io[i * k + j] = t[i * Kp + j];
-        }
+    if (main_io) st = download_states(c, main_io, dm, M, k, Kp, 1, c->stream, "download main window");
+    if (!st && !sp->high && blk_io) st = download_states(c, blk_io, db, B, k, Kp, 1, c->stream, "download blocked window");
+    if (st) {
+        release();
+        return st;
     }
 #undef OFP_HIP_R
     release();
@@ -2112,20 +2142,9 @@ ofp_status ofp_group_exchange(ofp_ctx* c, const ofp_group_spec* sp, int shares, 
     if (main_index && M) OFP_HIP(c, hipMemcpy(main_index, d_im, M * 8, hipMemcpyDeviceToHost), "download records");
     if (blocked_index && B)
         OFP_HIP(c, hipMemcpy(blocked_index, d_ib, B * 8, hipMemcpyDeviceToHost), "download records");
-    if ((main_res && M) || (blocked_res && B)) {
-        std::vector<uint32_t> t(std::max(M, B) * (size_t)Kp);
-        if (main_res && M) {
-            OFP_HIP(c, hipMemcpy(t.data(), d_rm, M * Kp * 4, hipMemcpyDeviceToHost), "download records");
-            for (uint64_t i = 0; i < M; ++i)
-                for (int j = 0; j < k; ++j) main_res[i * k + j] = t[i * Kp + j];
-        }
-        if (blocked_res && B) {
-            OFP_HIP(c, hipMemcpy(t.data(), d_rb, B * Kp * 4, hipMemcpyDeviceToHost), "download records");
-            for (uint64_t i = 0; i < B; ++i)
-                for (int j = 0; j < k; ++j) blocked_res[i * k + j] = t[i * Kp + j];
-        }
-    }
-    return OFP_OK;
+    if (main_res) st = download_states(c, main_res, d_rm, M, k, Kp, 1, c->stream, "download records");
+    if (!st && blocked_res) st = download_states(c, blocked_res, d_rb, B, k, Kp, 1, c->stream, "download records");
+    return st;
 }
 
 // ---- jobs: independent device-resident solves that overlap on the GPU ----
@@ -2222,6 +2241,7 @@ void ofp_destroy(ofp_ctx* c) {
     if (c->gfork) (void)hipEventDestroy(c->gfork);
     if (c->win) (void)hipFree(c->win);
     if (c->stage) (void)hipFree(c->stage);
+    if (c->io) (void)hipFree(c->io);
     if (c->ev0) (void)hipEventDestroy(c->ev0);
     if (c->ev1) (void)hipEventDestroy(c->ev1);
     if (c->stream) (void)hipStreamDestroy(c->stream);

@@ -32,6 +32,7 @@
 // Residues: uint32 mod p, additions only (every transfer coefficient is 1);
 // a + b mod p is one conditional subtract, written as a subtract with borrow
 // and a select (addm in ofp_cell_impl.h).
+#include <algorithm>
 #include <cstring>
 #include <vector>
 
@@ -309,6 +310,30 @@ hipError_t launch_fill_remote(uint32_t* main, uint64_t m0, uint64_t M, uint32_t*
     if (k < 1 || K < k) return hipErrorInvalidValue;
     hipLaunchKernelGGL(fill_remote_kernel, dim3(4096), dim3(256), 0, s, main, m0, M, blk, b0, B, K, k,
                        mods_dev, seed);
+    return hipGetLastError();
+}
+
+// One thread per (state, slot of the stride); packed reads and writes are coalesced,
+// the device words' too in the state-major layout.  Bound by the host copies around it.
+__global__ __launch_bounds__(256) void restride_kernel(uint32_t* dev, uint32_t* packed, uint64_t first, uint64_t n, int k,
+                                                       int Kp, int layout, int to_dev) {
+    const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
+    for (uint64_t t = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; t < n * (uint64_t)Kp; t += stride) {
+        const uint64_t i = t / (uint32_t)Kp;
+        const int j = (int)(t - i * (uint32_t)Kp);
+        uint32_t* d = dev + state_elem(layout, first + i, Kp, j);
+        if (to_dev) *d = j < k ? packed[i * (uint32_t)k + j] : 0u;
+        else if (j < k) packed[i * (uint32_t)k + j] = *d;
+    }
+}
+
+hipError_t launch_restride(uint32_t* dev, uint32_t* packed, uint64_t first, uint64_t n, int k, int Kp, int layout,
+                           bool to_dev, hipStream_t s) {
+    if (k < 1 || Kp < k) return hipErrorInvalidValue;
+    const uint64_t blocks = std::min<uint64_t>((n * (uint64_t)Kp + 255) / 256, 16384);
+    if (!blocks) return hipSuccess;
+    hipLaunchKernelGGL(restride_kernel, dim3((unsigned)blocks), dim3(256), 0, s, dev, packed, first, n, k, Kp, layout,
+                       to_dev ? 1 : 0);
     return hipGetLastError();
 }
 

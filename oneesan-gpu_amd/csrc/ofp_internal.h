@@ -88,6 +88,10 @@ hipError_t launch_cell_shard(const CellLaunch& a, bool wide_index, int threads, 
 hipError_t launch_fill_remote(uint32_t* main, uint64_t m0, uint64_t M, uint32_t* blk, uint64_t b0,
                               uint64_t B, int K, int k, const uint32_t* mods_dev, uint64_t seed,
                               hipStream_t s);
+// Copy states first..first+n-1 between dev (layout, stride Kp) and a packed buffer of n
+// states of k residues: to_dev writes dev (stride padding zero), else packed.
+hipError_t launch_restride(uint32_t* dev, uint32_t* packed, uint64_t first, uint64_t n, int k, int Kp, int layout,
+                           bool to_dev, hipStream_t s);
 // Set main[(index, j)] = 1 mod moduli[j] for j < k (interleave stride K) and, where
 // acc is given, its accs sums to zero.
 hipError_t launch_set_one(uint32_t* main, uint64_t index, int K, int k, int layout,
