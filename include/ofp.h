@@ -251,7 +251,7 @@ ofp_status ofp_set_low_cells(ofp_ctx* ctx, int low_cells, int low_kc);
 
 /* State layout for the next prepare/solve: 0 = tiles of 64 states (one
  * modulus of 64 consecutive states is 256 contiguous bytes), 1 = state-major
- * (the k residues of a state contiguous, stride padded to even).  No
+ * (the k residues of a state contiguous).  No
  * reference counterpart (the reference runs one modulus at a time); set by
  * the autotuner.  Invalidates the prepared state. */
 ofp_status ofp_set_layout(ofp_ctx* ctx, int layout);

@@ -63,7 +63,7 @@ struct ofp_ctx {
     int threads = 256;
     int blocks_per_cu = 32;
     int use_graphs = 1;
-    int layout = 1;  // 0: 64-state tiles, 1: state-major with even stride
+    int layout = 1;  // 0: 64-state tiles, 1: state-major
     int variant = 2;         // kernel variant (cell_kernel V parameter), set by the autotuner
     int low_cells = 0;       // cells p <= low_cells launch at most low_kc moduli at a time
     int low_kc = kMaxKC;
@@ -446,10 +446,9 @@ ofp_status enqueue_cells(ofp_ctx* c, Sweep& s, int p_hi, int p_lo, bool first_re
         if (cell_ev) OFP_HIP(c, hipEventRecord(cell_ev[2 * (p_hi - p)], s.stream), "event record");
         // moduli per launch: all (up to 16) at once, or fewer on the low cells,
         // whose scattered closure reads are latency-bound (fewer registers per
-        // thread -> more waves in flight).  Chunks keep an even offset.
+        // thread -> more waves in flight).
         int step = kMaxKC;
         if (p <= c->low_cells && c->low_kc < step) step = c->low_kc;
-        if (s.layout == 1 && s.K > 1 && (step & 1)) step = std::max(2, step - 1);
         for (int off = 0; off < s.K; off += step) {
             CellLaunch a{};
             a.main = s.main;
@@ -600,8 +599,7 @@ ofp_status enqueue_pair(ofp_ctx* c, Sweep& s, int p, bool reads_blk, int cap, in
             a.K = s.Kp;
             a.off = off;
             a.kc = kc;
-            // lanes past the k moduli (stride padding) compute with a valid modulus
-            for (int jj = 0; jj < kc; ++jj) a.mod[jj] = s.mods[off + jj < s.K ? off + jj : 0];
+            for (int jj = 0; jj < kc; ++jj) a.mod[jj] = s.mods[off + jj];
             a.xcd_shift = piece_shift(c->xcd_shift, cnt, c->threads);
             a.variant = c->pair_variant;
             hipStream_t ls = !par ? s.stream : (d == -1 || d == -2) ? s.par[0] : (d == 1 ? s.par[1] : s.stream);
@@ -877,8 +875,7 @@ ofp_status init_state(ofp_ctx* c, Sweep& s) {
 
 // Split k moduli into sweeps of at most g each (g >= 1): as few sweeps as
 // possible, sizes as equal as possible, and even sizes where that costs no
-// sweep (the state-major stride is padded to even, so an odd sweep carries
-// one idle slot).  Returns the number of sweeps; sizes[] gets the first cap.
+// sweep.  Returns the number of sweeps; sizes[] gets the first cap.
 int moduli_groups(int k, int g, int* sizes, int cap) {
     if (k < 1 || g < 1) return 0;
     const int groups = (k + g - 1) / g;
@@ -1490,7 +1487,7 @@ ofp_status ofp_shard_plan(ofp_ctx* c, const ofp_shard_spec* sp, ofp_shard_info* 
     info->first_main = m0;
     info->main_count = m1 - m0;
     info->low_cells = lc;
-    const int Kp = interleave_stride(1, sp->k);
+    const int Kp = window_stride(sp->k);
     info->state_bytes = (info->main_count + info->blocked_count) * (uint64_t)Kp * 4;
     info->kernel_s = 0;
     info->launches = 0;
@@ -1505,7 +1502,7 @@ ofp_status ofp_shard_sweep(ofp_ctx* c, const ofp_shard_spec* sp, ofp_shard_info*
     if (st) return st;
     for (int j = 0; j < sp->k; ++j)
         if (sp->moduli[j] < 2) return fail(c, OFP_E_ARG, "modulus must be in [2, 4294967295]");
-    const int W = sp->n + 1, k = sp->k, Kp = interleave_stride(1, k);
+    const int W = sp->n + 1, k = sp->k, Kp = window_stride(k);
     const uint64_t M = info->main_count, B = info->blocked_count;
     OFP_HIP(c, hipSetDevice(c->device), "hipSetDevice");
     const size_t mbytes = std::max<uint64_t>(M, 1) * Kp * 4, bbytes = std::max<uint64_t>(B, 1) * Kp * 4;
@@ -1626,7 +1623,7 @@ ofp_status ofp_group_plan(ofp_ctx* c, const ofp_group_spec* sp, ofp_group_info* 
     info->main_count = M;
     info->blocked_count = B;
     info->largest_group = big;
-    const int Kp = interleave_stride(1, sp->k);
+    const int Kp = window_stride(sp->k);
     info->state_bytes = (M + B) * (uint64_t)Kp * 4 + (uint64_t)sp->groups * kGroupTableBytes;
     info->low = L;
     info->cells = sp->high ? L : W - 1 - L;
@@ -1645,7 +1642,7 @@ ofp_status ofp_group_sweep(ofp_ctx* c, const ofp_group_spec* sp, ofp_group_info*
     for (uint32_t g = 0; g < G; ++g)
         if ((mc[g] >> 32) || (bc[g] >> 32))
             return fail(c, OFP_E_ARG, "a group of the window holds 2^32 or more words: use more low positions");
-    const int W = sp->n + 1, k = sp->k, Kp = interleave_stride(1, k), L = info->low;
+    const int W = sp->n + 1, k = sp->k, Kp = window_stride(k), L = info->low;
     const uint64_t M = info->main_count, B = info->blocked_count;
     std::vector<uint64_t> moff(G + 1, 0), boff(G + 1, 0);
     for (uint32_t g = 0; g < G; ++g) {
@@ -1956,7 +1953,7 @@ ofp_status ofp_group_exchange(ofp_ctx* c, const ofp_group_spec* sp, int shares, 
     if (!lw.valid || lw.n != sp->n || lw.k != sp->k || lw.low != L || lw.first != sp->first_group ||
         lw.groups != sp->groups)
         return fail(c, OFP_E_ARG, "no such LOW window in the context: sweep it with ofp_group_sweep first");
-    const int W = sp->n + 1, k = sp->k, Kp = interleave_stride(1, k), nf = W - 1 - L;
+    const int W = sp->n + 1, k = sp->k, Kp = window_stride(k), nf = W - 1 - L;
     if (nf > 16) return fail(c, OFP_E_ARG, "the exchange takes at most 16 fixed HIGH positions");
     const uint32_t NM = 1u << nf;
     // HIGH groups: word counts, the shares (consecutive masks, cut by main +

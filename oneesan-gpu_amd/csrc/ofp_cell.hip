@@ -274,8 +274,7 @@ hipError_t launch_cell(const CellLaunch& a, bool wide_index, int threads, int bl
     if (threads <= 0 || threads > 256 || (threads & 63) || blocks <= 0 || (blocks & 7))
         return hipErrorInvalidConfiguration;
     if (a.W < 2 || a.W > kMaxW || a.p < 1 || a.p > a.W - 1 || a.kc < 1 || a.kc > kMaxKC ||
-        a.off < 0 || a.off + a.kc > a.K || (a.layout != kAoSoA && a.layout != kAoS) ||
-        (a.layout == kAoS && a.K > 1 && ((a.K & 1) || (a.off & 1))))
+        a.off < 0 || a.off + a.kc > a.K || (a.layout != kAoSoA && a.layout != kAoS))
         return hipErrorInvalidValue;
     return wide_index ? launch_idx<uint64_t>(a, threads, blocks, s)
                       : launch_idx<uint32_t>(a, threads, blocks, s);
@@ -286,7 +285,7 @@ hipError_t launch_cell_capped(const CellLaunch& a, bool wide_index, int threads,
     if (threads <= 0 || threads > 256 || (threads & 63) || blocks <= 0 || (blocks & 7))
         return hipErrorInvalidConfiguration;
     if (a.W < 2 || a.W > kMaxW || a.p < 1 || a.p > a.W - 1 || a.kc < 1 || a.kc > kMaxKC || a.off < 0 ||
-        a.off + a.kc > a.K || a.layout != kAoS || (a.K > 1 && ((a.K & 1) || (a.off & 1))) || !a.dpc ||
+        a.off + a.kc > a.K || a.layout != kAoS || !a.dpc ||
         a.first != 0)
         return hipErrorInvalidValue;
     return wide_index ? launch_capped_idx<uint64_t>(a, threads, blocks, s)
@@ -298,7 +297,7 @@ hipError_t launch_cell_shard(const CellLaunch& a, bool wide_index, int threads, 
     if (threads <= 0 || threads > 256 || (threads & 63) || blocks <= 0 || (blocks & 7))
         return hipErrorInvalidConfiguration;
     if (a.W < 2 || a.W > kMaxW || a.p < 1 || a.p > a.W - 1 || a.layout != kAoS || a.off < 0 ||
-        a.off + a.kc > a.K || (a.K > 1 && ((a.K & 1) || (a.off & 1))) || !a.stray)
+        a.off + a.kc > a.K || !a.stray)
         return hipErrorInvalidValue;
     return wide_index ? launch_shard_idx<uint64_t>(a, threads, blocks, s)
                       : launch_shard_idx<uint32_t>(a, threads, blocks, s);

@@ -171,9 +171,8 @@ struct Sched {
 
 // State layouts.  kAoSoA: tiles of 64 states, modulus-major inside a tile
 // (a wave reading one modulus of 64 consecutive states reads 256 contiguous
-// bytes).  kAoS: state-major with an even stride, residues of one state
-// contiguous (one scattered state is one or two 64-byte sectors), read two
-// residues per 8-byte load.
+// bytes).  kAoS: state-major, residues of one state contiguous (one scattered state
+// is one or two 64-byte sectors), read four, two or one residues per load.
 enum Layout : int { kAoSoA = 0, kAoS = 1 };
 
 template <int L>
@@ -187,6 +186,26 @@ struct Vals {
     uint32_t v[KC];
 };
 
+// Words at 4-byte alignment: a record of an odd number of moduli is aligned to one
+// residue, which the 16- and 8-byte accesses of global memory need no more than.
+template <int N>
+struct __attribute__((packed, aligned(4))) Words {
+    uint32_t v[N];
+};
+template <int N>
+OFP_HD void load_words(const uint32_t* q, uint32_t* out) {
+    const Words<N> w = *reinterpret_cast<const Words<N>*>(q);
+#pragma unroll
+    for (int j = 0; j < N; ++j) out[j] = w.v[j];
+}
+template <int N>
+OFP_HD void store_words(uint32_t* q, const uint32_t* in) {
+    Words<N> w;
+#pragma unroll
+    for (int j = 0; j < N; ++j) w.v[j] = in[j];
+    *reinterpret_cast<Words<N>*>(q) = w;
+}
+
 template <int KC, int L>
 OFP_HD void load_vals(const uint32_t* __restrict__ base, uint64_t i, int K, int off, Vals<KC>& out) {
     const uint32_t* q = base + elem<L>(i, K, off);
@@ -194,13 +213,9 @@ OFP_HD void load_vals(const uint32_t* __restrict__ base, uint64_t i, int K, int 
 #pragma unroll
         for (int j = 0; j < KC; ++j) out.v[j] = q[j * kTile];
     } else {
-        const uint2* q2 = reinterpret_cast<const uint2*>(q);
 #pragma unroll
-        for (int j = 0; j + 1 < KC; j += 2) {
-            uint2 t = q2[j / 2];
-            out.v[j] = t.x;
-            out.v[j + 1] = t.y;
-        }
+        for (int j = 0; j + 3 < KC; j += 4) load_words<4>(q + j, out.v + j);
+        if constexpr (KC & 2) load_words<2>(q + (KC & ~3), out.v + (KC & ~3));
         if constexpr (KC & 1) out.v[KC - 1] = q[KC - 1];
     }
 }
@@ -211,9 +226,9 @@ OFP_HD void store_vals(uint32_t* __restrict__ base, uint64_t i, int K, int off, 
 #pragma unroll
         for (int j = 0; j < KC; ++j) q[j * kTile] = in.v[j];
     } else {
-        uint2* q2 = reinterpret_cast<uint2*>(q);
 #pragma unroll
-        for (int j = 0; j + 1 < KC; j += 2) q2[j / 2] = make_uint2(in.v[j], in.v[j + 1]);
+        for (int j = 0; j + 3 < KC; j += 4) store_words<4>(q + j, in.v + j);
+        if constexpr (KC & 2) store_words<2>(q + (KC & ~3), in.v + (KC & ~3));
         if constexpr (KC & 1) q[KC - 1] = in.v[KC - 1];
     }
 }

@@ -37,16 +37,11 @@ using cell::Quad;
 template <int KC>
 __device__ __forceinline__ void load_rec(const uint32_t* base, uint64_t i, int K, int off, uint32_t (&v)[KC]) {
     const uint32_t* q = base + i * (uint64_t)(uint32_t)K + (uint32_t)off;
-    if constexpr (KC == 1) {
-        v[0] = q[0];
+    if (off + KC <= K) {
+        cell::load_words<KC>(q, v);
     } else {
 #pragma unroll
-        for (int j = 0; j < KC; j += 2) {
-            uint2 t = make_uint2(0u, 0u);
-            if (j == 0 || off + j < K) t = *reinterpret_cast<const uint2*>(q + j);
-            v[j] = t.x;
-            v[j + 1] = t.y;
-        }
+        for (int j = 0; j < KC; ++j) v[j] = off + j < K ? q[j] : 0u;
     }
 }
 
@@ -254,9 +249,7 @@ __global__ __launch_bounds__(256) void glue_gather_kernel(GlueLaunch a) {
     uint32_t* out = entry(a, t, l);
     const uint64_t r = (uint64_t)word_rank<Idx>(D, reversed_mask(occ, a.W), labels_of(b, g.m, l), 31);
     const uint32_t* src = a.main + r * (uint64_t)(uint32_t)a.K;
-    if (a.K == 1) out[0] = src[0];
-    else
-        for (int j = 0; j < a.K; j += 2) *reinterpret_cast<uint2*>(out + j) = *reinterpret_cast<const uint2*>(src + j);
+    for (int j = 0; j < a.K; ++j) out[j] = src[j];
 }
 
 // One level down: entry v of every array of M - 2 strands = the sum over the
@@ -294,13 +287,9 @@ __global__ __launch_bounds__(256) void glue_pull_kernel(GlueLaunch a, uint32_t a
         for (int j = 0; j < KC; ++j) sum[j] = addm(sum[j], e[j], mod[j]);
     });
     uint32_t* out = entry(a, t, a.to + node * rows + l) + off;
-    if constexpr (KC == 1) {
-        out[0] = sum[0];
-    } else {
-        *reinterpret_cast<uint2*>(out) = make_uint2(sum[0], sum[1]);
-        if constexpr (KC == 4)
-            if (off + 2 < a.K) *reinterpret_cast<uint2*>(out + 2) = make_uint2(sum[2], sum[3]);
-    }
+#pragma unroll
+    for (int j = 0; j < KC; ++j)
+        if (off + j < a.K) out[j] = sum[j];
 }
 
 // One thread per (task, upper word): its arcs removed down to kTabStrands, its list

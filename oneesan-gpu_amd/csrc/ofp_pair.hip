@@ -66,7 +66,7 @@ hipError_t launch_d(const pair::PairLaunch& a, int threads, int blocks, hipStrea
 template <int KC, typename Idx>
 hipError_t launch_gf(const pair::PairLaunch& a, int threads, int blocks, hipStream_t s) {
     if (a.cap > 0) return launch_d<KC, Idx, 0, 2, true>(a, threads, blocks, s);
-    if constexpr (KC >= 14) {
+    if constexpr (KC == 14 || KC == 16) {
         switch (a.variant & 3) {
             case 1: return launch_d<KC, Idx, 1, 2>(a, threads, blocks, s);
             case 2: return launch_d<KC, Idx, 0, 3>(a, threads, blocks, s);
@@ -135,30 +135,12 @@ uint64_t pair_class_count(int W, int p, int d, int cap) {
 hipError_t launch_pair(const pair::PairLaunch& a, bool wide, int threads, int blocks, hipStream_t s) {
     if (a.p < 2 || a.p > a.W - 1 || a.d < -3 || a.d > 3 || a.kc < 1 || a.off + a.kc > a.K || a.cap < 0 || a.cap > kPairCaps)
         return hipErrorInvalidValue;
-    if (wide) {
-        switch (a.kc) {
-            case 1: return launch_gf<1, uint64_t>(a, threads, blocks, s);
-            case 2: return launch_gf<2, uint64_t>(a, threads, blocks, s);
-            case 4: return launch_gf<4, uint64_t>(a, threads, blocks, s);
-            case 6: return launch_gf<6, uint64_t>(a, threads, blocks, s);
-            case 8: return launch_gf<8, uint64_t>(a, threads, blocks, s);
-            case 10: return launch_gf<10, uint64_t>(a, threads, blocks, s);
-            case 12: return launch_gf<12, uint64_t>(a, threads, blocks, s);
-            case 14: return launch_gf<14, uint64_t>(a, threads, blocks, s);
-            case 16: return launch_gf<16, uint64_t>(a, threads, blocks, s);
-            default: return hipErrorInvalidValue;
-        }
-    }
     switch (a.kc) {
-        case 1: return launch_gf<1, uint32_t>(a, threads, blocks, s);
-        case 2: return launch_gf<2, uint32_t>(a, threads, blocks, s);
-        case 4: return launch_gf<4, uint32_t>(a, threads, blocks, s);
-        case 6: return launch_gf<6, uint32_t>(a, threads, blocks, s);
-        case 8: return launch_gf<8, uint32_t>(a, threads, blocks, s);
-        case 10: return launch_gf<10, uint32_t>(a, threads, blocks, s);
-        case 12: return launch_gf<12, uint32_t>(a, threads, blocks, s);
-        case 14: return launch_gf<14, uint32_t>(a, threads, blocks, s);
-        case 16: return launch_gf<16, uint32_t>(a, threads, blocks, s);
+#define OFP_KC(n) \
+    case n: return wide ? launch_gf<n, uint64_t>(a, threads, blocks, s) : launch_gf<n, uint32_t>(a, threads, blocks, s);
+        OFP_KC(1) OFP_KC(2) OFP_KC(3) OFP_KC(4) OFP_KC(5) OFP_KC(6) OFP_KC(7) OFP_KC(8)
+        OFP_KC(9) OFP_KC(10) OFP_KC(11) OFP_KC(12) OFP_KC(13) OFP_KC(14) OFP_KC(15) OFP_KC(16)
+#undef OFP_KC
         default: return hipErrorInvalidValue;
     }
 }
