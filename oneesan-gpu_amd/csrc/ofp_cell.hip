@@ -44,13 +44,6 @@ namespace {
 
 using namespace cell;
 
-// Copy the first kLdsRows x C entries of a kDpRows x kDpCols table into LDS
-// (row stride C there).
-template <int C, typename T>
-__device__ void load_table(T* dst, const T* src) {
-    for (int t = threadIdx.x; t < kLdsRows * C; t += blockDim.x) dst[t] = src[(t / C) * kDpCols + t % C];
-}
-
 // Work distribution: the blocked range is cut into chunks of blockDim.x words;
 // workgroup g runs on XCD g%8 (round-robin dispatch).  The chunks are dealt to
 // the XCDs in pieces of 2^shift consecutive chunks, round-robin (piece i to XCD
@@ -63,7 +56,7 @@ template <int KC, typename Idx, int L, int V>
 __global__ __launch_bounds__(256) void cell_kernel(CellLaunch a) {
     __shared__ Quad<Idx> tab[kLdsRows][LdsCols<Idx>::value];
     const Quad<Idx>* g = (const Quad<Idx>*)a.dp;
-    load_table<LdsCols<Idx>::value>(&tab[0][0], g);
+    load_table<LdsCols<Idx>::value, kDpCols>(&tab[0][0], g, a.W);
     __syncthreads();
     Tab<Idx> T{tab};
     const Direct<KC, L, Idx> mem{a.main, a.blk, a.K, a.off};
@@ -126,7 +119,7 @@ __global__ __launch_bounds__(256) void cell_sorted_kernel(CellLaunch a) {
     __shared__ Decoded<Idx> slot[256];
     __shared__ uint32_t cnt[2][4];
     const Quad<Idx>* g = (const Quad<Idx>*)a.dp;
-    load_table<LdsCols<Idx>::value>(&tab[0][0], g);
+    load_table<LdsCols<Idx>::value, kDpCols>(&tab[0][0], g, a.W);
     __syncthreads();
     Tab<Idx> T{tab};
     const Direct<KC, kAoS, Idx> mem{a.main, a.blk, a.K, a.off};
@@ -138,7 +131,7 @@ template <int KC, typename Idx, int V>
 __global__ __launch_bounds__(256) void cell_shard_kernel(CellLaunch a) {
     __shared__ Quad<Idx> tab[kLdsRows][LdsCols<Idx>::value];
     const Quad<Idx>* g = (const Quad<Idx>*)a.dp;
-    load_table<LdsCols<Idx>::value>(&tab[0][0], g);
+    load_table<LdsCols<Idx>::value, kDpCols>(&tab[0][0], g, a.W);
     __syncthreads();
     Tab<Idx> T{tab};
     Windowed<KC> mem;
@@ -170,8 +163,8 @@ __global__ __launch_bounds__(256) void cell_capped_kernel(CellLaunch a) {
     __shared__ Pair<Idx> ctab[kLdsRows][LdsCols<Idx>::value];
     const Quad<Idx>* g = (const Quad<Idx>*)a.dp;
     const Pair<Idx>* gc = (const Pair<Idx>*)a.dpc;
-    load_table<LdsCols<Idx>::value>(&tab[0][0], g);
-    load_table<LdsCols<Idx>::value>(&ctab[0][0], gc);
+    load_table<LdsCols<Idx>::value, kDpCols>(&tab[0][0], g, a.W);
+    load_table<LdsCols<Idx>::value, kDpCols>(&ctab[0][0], gc, a.W);
     __syncthreads();
     Tab<Idx> T{tab};
     const Direct<KC, kAoS, Idx> mem{a.main, a.blk, a.K, a.off};

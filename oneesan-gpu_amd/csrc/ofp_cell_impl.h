@@ -119,6 +119,10 @@ struct LdsCols {
     static constexpr int value = sizeof(Idx) == 8 ? 22 : kDpCols;
 };
 
+// Columns a row of width W reads: its words' heights are at most (W+1)/2 (one open
+// bracket more than positions left to close it, entered at 1), the scans read two above.
+OFP_HD int used_cols(int W) { return (W + 1) / 2 + 3; }
+
 template <typename Idx>
 struct Tab {
     const Quad<Idx> (*q)[LdsCols<Idx>::value];
@@ -145,6 +149,18 @@ struct Tab {
         return step_z(e.zn, e.zc, r, contrib);
     }
 };
+
+#ifdef __HIP__
+// The entries a row of width W reads, rows 0..W-1 of a table (row stride S in memory, C
+// in LDS; 32 threads per row).  A small launch is little more than this: n=15 at 3
+// moduli, 123 launches, with whole tables 1.77 ms, see the launch notes in ofp_cell.hip.
+template <int C, int S, typename T>
+__device__ __forceinline__ void load_table(T* dst, const T* src, int W) {
+    const int col = threadIdx.x & 31, cols = used_cols(W);
+    if (col >= cols) return;
+    for (int r = threadIdx.x >> 5; r < W; r += blockDim.x >> 5) dst[r * C + col] = src[r * S + col];
+}
+#endif
 
 // Chunk schedule of one workgroup over n words in chunks of bdim (see the
 // work-distribution note in ofp_cell.hip).

@@ -17,11 +17,6 @@ namespace {
 
 using namespace cell;
 
-template <int C, typename T>
-__device__ void load_rows(T* dst, const T* src) {
-    for (int t = threadIdx.x; t < kLdsRows * C; t += blockDim.x) dst[t] = src[t];
-}
-
 // MB: workgroups of 256 per CU the register allocation must allow (2: at most
 // 256 VGPRs, no spills at 14 moduli; 3: at most 168, with spills).
 // Capped: the classes of a height-capped pass (a.cap).
@@ -31,8 +26,8 @@ __global__ __launch_bounds__(256, MB) void pair_kernel(pair::PairLaunch a) {
     __shared__ Quad<Idx> tab[kLdsRows][C];
     __shared__ Pair<Idx> ctab[kLdsRows][C];
     const Quad<Idx>* g = (const Quad<Idx>*)a.dp;
-    for (int t = threadIdx.x; t < kLdsRows * C; t += blockDim.x) (&tab[0][0])[t] = g[(t / C) * kDpCols + t % C];
-    load_rows<C>(&ctab[0][0], (const Pair<Idx>*)a.ct);
+    load_table<C, kDpCols>(&tab[0][0], g, a.W);
+    load_table<C, C>(&ctab[0][0], (const Pair<Idx>*)a.ct, a.W);
     __syncthreads();
     Tab<Idx> T{tab};
     const pair::Io<KC, Idx> io{a.main_in, a.blk_in, a.main_out, a.blk_out, a.K, a.off};
