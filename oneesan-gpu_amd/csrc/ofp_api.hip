@@ -33,6 +33,11 @@ struct Sweep {
     uint32_t* main = nullptr;
     uint32_t* blk = nullptr;
     size_t main_cap = 0, blk_cap = 0;  // bytes allocated
+    // small states: a second pair of arrays, as large, that a pair pass goes to (and the
+    // two pairs change places); null: none
+    uint32_t* main2 = nullptr;
+    uint32_t* blk2 = nullptr;
+    bool whole = false;  // both pairs started from one state (init_state)
     uint32_t* mods_dev = nullptr;
     int mods_cap = 0;
     int n = 0, W = 0, K = 0, Kp = 0;  // k moduli, interleave stride Kp
@@ -234,10 +239,12 @@ void free_sweep(Sweep& s) {
     s.pfork = nullptr;
     sweep_free(s, s.main);
     sweep_free(s, s.blk);
+    sweep_free(s, s.main2);
+    sweep_free(s, s.blk2);
     sweep_free(s, s.mods_dev);
     sweep_free(s, s.acc);
     sweep_free(s, s.gscratch);
-    s.main = s.blk = s.mods_dev = s.gscratch = nullptr;
+    s.main = s.blk = s.main2 = s.blk2 = s.mods_dev = s.gscratch = nullptr;
     s.acc = nullptr;
     s.main_cap = s.blk_cap = s.gscratch_cap = 0;
     s.mods_cap = 0;
@@ -315,6 +322,31 @@ struct Carve {
 // 64-bit above or when forced).
 bool pairs_apply(const ofp_ctx* c, int n) { return c->pair_rows != 0 && c->layout == 1 && n >= 2; }
 
+// Words from which two cells run as one pair pass in place unless asked otherwise: a
+// pass is up to five launches, whose fixed times outweigh the bytes saved on few words.
+// Whole solves, cells alone against passes: n=16 (5.7e6 words) 3.19 against 4.06 ms at
+// one modulus, 7.85 against 8.33 at eight; n=17 (1.6e7) 6.82 against 6.65 and 24.5
+// against 22.9; n=14 (7e5) 1.05 against 1.90, 2.29 against 3.52.
+constexpr uint64_t kPairWords = 1ull << 23;
+
+// Residues below which two cells run as one launch to a second pair of arrays
+// (ofp_pair_whole.hip), unless asked otherwise: both pairs then fit the 256 MB last-level
+// cache, and the words such a pass copies cost less than the launches it saves.  Whole
+// solves, ms, without and with: n=12 at one modulus 0.64, 0.55; n=14 at 4 1.21, 1.18;
+// n=15 at 8 (1.6e7 residues) 2.70, 2.32; n=16 at one 3.06, 2.06; at 5 (2.8e7) 4.85, 4.27;
+// at 8 (4.5e7) 6.45, 6.88; n=17 at one 6.26, 4.77; at 2 (3.2e7) 7.51, 6.38; at 3 (4.8e7)
+// 8.95, 10.0; n=18 at one (4.4e7) 14.5, 15.8.  More than kWholeKC moduli would take two
+// launches a pass, each with the index math of one: n=15 at 12 3.70, 5.01.
+constexpr uint64_t kWholeWords = 1ull << 25;
+
+// Whether n at k moduli runs such passes: 32-bit ranks, pair passes left to the library.
+bool whole_size(const ofp_ctx* c, int n, int k) {
+    uint64_t nm, nb;
+    return c->pair_rows < 0 && c->layout == 1 && c->index_bits != 64 && n >= 2 && n <= 22 && counts(n, &nm, &nb) &&
+           k <= kWholeKC && (nm + nb) * k < kWholeWords;
+}
+bool whole_ready(const ofp_ctx* c, const Sweep& s) { return s.whole && s.layout == 1 && whole_size(c, s.n, s.K); }
+
 ofp_status ensure_state(ofp_ctx* c, Sweep& s, int n, const uint32_t* moduli, int k) {
     uint64_t nm, nb;
     if (!counts(n, &nm, &nb)) return fail(c, OFP_E_RANGE, "n must be in 1..27");
@@ -329,7 +361,9 @@ ofp_status ensure_state(ofp_ctx* c, Sweep& s, int n, const uint32_t* moduli, int
         drop_graph(s);
         sweep_free(s, s.main);
         sweep_free(s, s.blk);
-        s.main = s.blk = nullptr;
+        sweep_free(s, s.main2);
+        sweep_free(s, s.blk2);
+        s.main = s.blk = s.main2 = s.blk2 = nullptr;
         s.main_cap = s.blk_cap = 0;
         release_window(c);
         size_t fr = 0, tot = 0;
@@ -341,6 +375,12 @@ ofp_status ensure_state(ofp_ctx* c, Sweep& s, int n, const uint32_t* moduli, int
         OFP_HIP(c, sweep_alloc(s, (void**)&s.blk, bb), "allocate blocked state");
         s.main_cap = mb;
         s.blk_cap = bb;
+    }
+    s.whole = false;
+    if (whole_size(c, n, k)) {  // without the room, as above these sizes
+        if (!s.main2 && sweep_alloc(s, (void**)&s.main2, s.main_cap) != hipSuccess) s.main2 = nullptr;
+        if (!s.blk2 && sweep_alloc(s, (void**)&s.blk2, s.blk_cap) != hipSuccess) s.blk2 = nullptr;
+        (void)hipGetLastError();
     }
     if (s.mods_cap < k) {
         sweep_free(s, s.mods_dev);
@@ -521,12 +561,6 @@ ofp_status pass_streams(ofp_ctx* c, Sweep& s) {
     return OFP_OK;
 }
 
-// Words from which two cells run as one pair pass unless asked otherwise: a pass is
-// up to five launches, whose fixed times outweigh the bytes saved on few words.
-// Whole solves, cells alone against passes: n=16 (5.7e6 words) 3.19 against 4.06 ms at
-// one modulus, 7.85 against 8.33 at eight; n=17 (1.6e7) 6.82 against 6.65 and 24.5
-// against 22.9; n=14 (7e5) 1.05 against 1.90, 2.29 against 3.52.
-constexpr uint64_t kPairWords = 1ull << 23;
 // State bytes a pass covers from which its launches run side by side on three
 // streams.  Below, the fork and join cost more than the overlap gives: the capped
 // rows of an n=18 solve of one modulus (at most 177 MB) 5.17 ms with them, 4.17
@@ -543,11 +577,48 @@ uint64_t covered_words(const Sweep& s, int cap) {
 // height cap `cap`.
 bool pair_at(const ofp_ctx* c, const Sweep& s, int p, int p_lo, int cap) {
     const uint32_t mask = c->pair_mask ? c->pair_mask : default_pair_mask(std::min(s.K, c->pair_kc));
-    return p - 1 >= p_lo && p >= 2 && ((mask >> p) & 1u) && (c->pair_rows > 0 || covered_words(s, cap) >= kPairWords);
+    if (p - 1 < p_lo || p < 2) return false;
+    if (whole_ready(c, s)) return true;
+    return ((mask >> p) & 1u) && (c->pair_rows > 0 || covered_words(s, cap) >= kPairWords);
+}
+
+// A small pair pass over cells p and p-1: one launch per kWholeKC moduli, to the other
+// pair of arrays, which take the state's place.
+ofp_status enqueue_pair_whole(ofp_ctx* c, Sweep& s, int p, bool reads_blk, int cap, int* launches) {
+    const size_t tb = class_table_bytes(false);
+    pair::PairLaunch a{};
+    a.main_in = s.main;
+    a.blk_in = s.blk;
+    a.main_out = s.main2;
+    a.blk_out = s.blk2;
+    a.dp = c->dp32;
+    a.ct = static_cast<const char*>(c->ct32) + tb * (size_t)(cap * kMaxW + p) * 7;
+    a.ct_bytes = (uint32_t)tb;
+    a.W = s.W;
+    a.p = p;
+    a.read_blk = reads_blk ? 1 : 0;
+    a.cap = cap;
+    a.K = s.Kp;
+    for (int d = -3; d <= 3; ++d) {
+        a.count[d + 3] = (uint32_t)pair_class_count(s.W, p, d, cap);
+        a.block[d + 4] = a.block[d + 3] + (a.count[d + 3] + c->threads - 1) / c->threads;
+    }
+    for (int off = 0; off < s.Kp; off += kWholeKC) {
+        a.off = off;
+        a.kc = std::min(kWholeKC, s.Kp - off);
+        for (int j = 0; j < a.kc; ++j) a.mod[j] = s.mods[off + j];
+        const hipError_t e = launch_pair_whole(a, c->threads, s.stream);
+        if (e != hipSuccess) return hip_fail(c, e, "pair pass launch");
+        if (launches) ++*launches;
+    }
+    std::swap(s.main, s.main2);
+    std::swap(s.blk, s.blk2);
+    return OFP_OK;
 }
 
 // One pair pass over cells p and p-1 (cap > 0: over the classes at heights <= cap).
 ofp_status enqueue_pair(ofp_ctx* c, Sweep& s, int p, bool reads_blk, int cap, int* launches) {
+    if (whole_ready(c, s)) return enqueue_pair_whole(c, s, p, reads_blk, cap, launches);
     const int W = s.W;
     const bool wide = s.W > 23 || c->index_bits == 64;
     const size_t tb = class_table_bytes(wide);
@@ -648,7 +719,7 @@ ofp_status full_rows(ofp_ctx* c, Sweep& s, int rows, int* launches) {
     auto row = [&](int* l) {
         return pairs ? enqueue_pairs(c, s, s.W - 1, 1, false, l) : enqueue_cells(c, s, s.W - 1, 1, false, l);
     };
-    if (!c->use_graphs || s.fixed) {
+    if (!c->use_graphs || s.fixed || whole_ready(c, s)) {  // (small passes change the arrays' places)
         for (int r = 0; r < rows; ++r) {
             ofp_status st = row(launches);
             if (st) return st;
@@ -859,6 +930,27 @@ ofp_status run_rows(ofp_ctx* c, Sweep& s, int rows, int* launches, RowTimes* tim
 // Zero main and blocked and place the start word R at position W-1 (rank
 // H_DP[W-1][1]) with residue 1 (fullmate_dropN_batch.cu:508-511).
 ofp_status init_state(ofp_ctx* c, Sweep& s) {
+    s.whole = s.main2 && s.blk2 && s.layout == 1 && whole_size(c, s.n, s.K);
+    if (s.whole) {  // both pairs of arrays: capped passes leave words above their cap unwritten
+        WholeInit a{};
+        const uint64_t mw = padded_states(s.nmain) * (uint64_t)s.Kp, bw = padded_states(s.nblk ? s.nblk : 1) * (uint64_t)s.Kp;
+        a.array[0] = s.main;
+        a.array[1] = s.blk;
+        a.array[2] = s.main2;
+        a.array[3] = s.blk2;
+        a.words[0] = a.words[2] = mw;
+        a.words[1] = a.words[3] = bw;
+        a.start = dp_at(s.W - 1, 1) * (uint64_t)s.Kp;
+        a.acc = s.acc;
+        a.k = s.K;
+        a.accs = glue::kAccWords * s.K;
+        a.mods = s.mods_dev;
+        if (!a.mods)
+            for (int j = 0; j < s.K; ++j) a.mod[j] = s.mods[j];
+        s.row = 0;
+        OFP_HIP(c, launch_init_whole(a, s.stream), "init kernel");
+        return OFP_OK;
+    }
     OFP_HIP(c, hipMemsetAsync(s.main, 0, padded_states(s.nmain) * (size_t)s.Kp * 4, s.stream), "zero main state");
     // capped cells leave the blocked words above their cap untouched: those must read as zero
     OFP_HIP(c, hipMemsetAsync(s.blk, 0, padded_states(s.nblk ? s.nblk : 1) * (size_t)s.Kp * 4, s.stream),
@@ -1404,6 +1496,9 @@ ofp_status ofp_solve_static(ofp_ctx* c, int n, const uint32_t* moduli, int k, ui
     s.blk = s.main + mb / sizeof(uint32_t);  // mb is a multiple of 256 bytes (64 states x 4 B)
     s.main_cap = mb;
     s.blk_cap = bb;
+    const bool two = whole_size(c, n, k) && 2 * (mb + bb) <= kStaticStateBytes;  // room for the second pair
+    s.main2 = two ? s.blk + bb / sizeof(uint32_t) : nullptr;
+    s.blk2 = two ? s.main2 + mb / sizeof(uint32_t) : nullptr;
     s.mods_dev = nullptr;  // the start word takes the moduli by value
     s.acc = c->static_acc;
     s.mods.assign(moduli, moduli + k);
@@ -1420,7 +1515,7 @@ ofp_status ofp_solve_static(ofp_ctx* c, int n, const uint32_t* moduli, int k, ui
     st = run_rows(c, s, s.W, &launches, nullptr, half_ready(c, s));
     if (st) return st;
     st = read_main(c, s, 0, residues_out, k);
-    s.main = s.blk = nullptr;
+    s.main = s.blk = s.main2 = s.blk2 = nullptr;
     return st;
 }
 

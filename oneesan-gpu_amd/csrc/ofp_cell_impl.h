@@ -152,8 +152,9 @@ struct Tab {
 
 #ifdef __HIP__
 // The entries a row of width W reads, rows 0..W-1 of a table (row stride S in memory, C
-// in LDS; 32 threads per row).  A small launch is little more than this: n=15 at 3
-// moduli, 123 launches, with whole tables 1.77 ms, see the launch notes in ofp_cell.hip.
+// in LDS; 32 threads per row).  Copying whole tables, a workgroup of n=17 loads 4 times
+// what it reads: solves at one modulus 6.40 ms, now 6.27 (n=18 14.8 and 14.5; where
+// launches are the bound, n <= 15, no difference).
 template <int C, int S, typename T>
 __device__ __forceinline__ void load_table(T* dst, const T* src, int W) {
     const int col = threadIdx.x & 31, cols = used_cols(W);

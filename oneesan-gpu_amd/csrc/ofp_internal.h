@@ -116,6 +116,21 @@ size_t class_table_bytes(bool wide);
 uint64_t pair_class_count(int W, int p, int d, int cap);
 // One pair-pass launch (a.kc in 1..16 moduli).
 hipError_t launch_pair(const pair::PairLaunch& a, bool wide_index, int threads, int blocks, hipStream_t s);
+// A pair pass from main_in / blk_in to main_out / blk_out in one launch (32-bit ranks,
+// at most kWholeKC moduli; ofp_pair_whole.hip).
+constexpr int kWholeKC = 8;
+hipError_t launch_pair_whole(const pair::PairLaunch& a, int threads, hipStream_t s);
+// A fresh state for such passes: the arrays (words: multiples of 4) zero but the k
+// residues from element `start` of array 0, which get 1 mod their modulus; accs sums zero.
+struct WholeInit {
+    uint32_t* array[4];
+    uint64_t words[4], start;
+    uint64_t* acc;
+    int k, accs;
+    const uint32_t* mods;  // on the device, or null: mod
+    uint32_t mod[kMaxKC];
+};
+hipError_t launch_init_whole(const WholeInit& a, hipStream_t s);
 
 // ---- exchange between the two placements of a row (ofp_exchange.hip) ----
 // A tile: `len` consecutive words of one group of a LOW window (local ranks

@@ -9,6 +9,8 @@
 // still hold their values from before the pass when it reads them (launch
 // order d = -1, 0, 1, then -2, 2), so the launches need no atomics and no
 // second copy of the state.
+#include <algorithm>
+
 #include "ofp_pair_impl.h"
 
 namespace ofp {
@@ -120,11 +122,32 @@ hipError_t launch_class_tables(bool wide, void* out, hipStream_t s) {
     return hipGetLastError();
 }
 
+// The prefixes P' that end at height h, times the suffixes S' entered at h + d, summed
+// over h: pair::class_count without a table of its own per launch (seven a pass).
 uint64_t pair_class_count(int W, int p, int d, int cap) {
-    uint64_t d0[kDpRows][kDpCols];
-    if (cap > 0) build_capped_table(cap, d0);
-    else build_height_table(d0);
-    return pair::class_count(d0, W, p, d, cap);
+    struct Words {
+        uint64_t down[kPairCaps + 1][kDpRows][kDpCols];  // words of w positions from h to 0
+        uint64_t up[kPairCaps + 1][kDpRows][kDpCols];    // words of w positions from 1 to h
+        Words() {
+            for (int c = 0; c <= kPairCaps; ++c) {
+                if (c > 0) build_capped_table(c, down[c]);
+                else build_height_table(down[c]);
+                const int top = c > 0 ? c : kDpCols - 1;
+                for (int w = 0; w < kDpRows; ++w)
+                    for (int h = 0; h < kDpCols; ++h)
+                        up[c][w][h] = h > top ? 0
+                                      : w == 0 ? (h == 1)
+                                               : up[c][w - 1][h] + (h > 0 ? up[c][w - 1][h - 1] : 0) +
+                                                     (h < top ? up[c][w - 1][h + 1] : 0);
+            }
+        }
+    };
+    static const Words words;  // the same for every context
+    uint64_t n = 0;
+    if (p < 2 || p > W - 1) return 0;
+    for (int h = std::max(0, -d); h + std::max(0, d) < kDpCols; ++h)
+        n += words.up[cap][W - 1 - p][h] * words.down[cap][p - 2][h + d];
+    return n;
 }
 
 hipError_t launch_pair(const pair::PairLaunch& a, bool wide, int threads, int blocks, hipStream_t s) {

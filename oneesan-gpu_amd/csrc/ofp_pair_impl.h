@@ -146,6 +146,10 @@ struct PairLaunch {
     int K, off, kc;    // interleave stride, first modulus, moduli in this launch
     int xcd_shift;
     int variant;        // kernel variant: bit 0 = gathers first (pair_body's GF), bit 1 = tighter registers
+    // one launch over every window change d = -3..3 (launch_pair_whole): classes, first
+    // workgroup and class table (ct + (d + 3) * ct_bytes) of each
+    uint32_t count[7], block[8];
+    uint32_t ct_bytes;
     uint32_t mod[kMaxKC];
 };
 
@@ -362,8 +366,10 @@ OFP_HD void closures_after(const Tab<Idx>& T, int W, int p, const Class<Idx>& k,
 // The pass over one class of window change D.  GF = 0: the class's words are
 // loaded first and the closure scans run while they are in flight; GF = 1: the
 // closure sums (the parts read from memory) are gathered first and the class's
-// words loaded after them, so that fewer values are live during the scans.
-template <int KC, typename Idx, int D, int GF = 0>
+// words loaded after them, so that fewer values are live during the scans.  Whole:
+// the pass goes from one pair of arrays to another (io), so the words it keeps are
+// stored too; then no class reads what another writes, in any order.
+template <int KC, typename Idx, int D, int GF = 0, bool Whole = false>
 OFP_HD void pair_body(const PairLaunch& a, const Tab<Idx>& T, const Class<Idx>& k, const Io<KC, Idx>& io) {
     using S = Slots<D>;
     const int W = a.W, p = a.p, h = k.h;
@@ -472,7 +478,7 @@ OFP_HD void pair_body(const PairLaunch& a, const Tab<Idx>& T, const Class<Idx>& 
 
     // ---- cell p-1: orbits of the blocked words (u, x') (u at p, x' at p-2) ----
     auto store_main = [&](int i) {
-        if (pm[i]) io.sm(im[i], m[i]);
+        if (!Whole && pm[i]) io.sm(im[i], m[i]);
     };
     auto store_blk = [&](int i) {
         if (p - 1 >= 2 && pb[i]) io.sb(ib[i], bl[i]);
@@ -538,6 +544,11 @@ OFP_HD void pair_body(const PairLaunch& a, const Tab<Idx>& T, const Class<Idx>& 
         if (code == 0 * 9 + 1 * 3 + 1 || code == 0 * 9 + 1 * 3 + 2 || code == 0 * 9 + 2 * 3 + 2 ||
             code == 2 * 9 + 1 * 3 + 1 || code == 2 * 9 + 1 * 3 + 2)
             store_main(i);
+    }
+    if constexpr (Whole) {
+#pragma unroll
+        for (int i = 0; i < S::NM; ++i)
+            if (pm[i]) io.sm(im[i], m[i]);
     }
 }
 
