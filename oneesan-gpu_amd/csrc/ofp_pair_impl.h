@@ -267,100 +267,152 @@ OFP_HD void vadd(Vals<KC>& acc, const Vals<KC>& x, const uint32_t* mod) {
     for (int j = 0; j < KC; ++j) acc.v[j] = addm(acc.v[j], x.v[j], mod[j]);
 }
 
-// Closure sources of the x=N word of cell p-1 in other classes, at their value
-// after cell p, added into acc (their classes have |d| >= 2 or leave them
-// unchanged, see the head of this file).  u = the symbol at main position p (the lowest
-// of the cell-(p-1) prefix P'' = (P', u)), hq = h + dh(u).
-//   LL: [P', u, L, L, S*] (S* = S' with a top-level L turned into R), scan of S';
-//   RR: [P'*, u, R, R, S'] (P'* = P' with a top-level R turned into L), scan of
-//       P' (the in-class source with u itself flipped is added by the caller).
-// u = N: the source was an NL / NR target of cell p and is rebuilt from old
-// (its blocked term only when the blocked input of cell p is valid).
-template <int KC, typename Idx>
-OFP_HD void closures_after(const Tab<Idx>& T, int W, int p, const Class<Idx>& k, int u, bool read_blk,
-                           const Io<KC, Idx>& io, Vals<KC>& acc, const uint32_t* mod) {
-    const int h = k.h, hq = h + dh(u);
-    const Idx mbq = k.mainbase + mcontrib(T, p, u, h);  // main contribution of P''
-    Vals<KC> t;
-    // LL (cell p-1 >= 3): scan S' downwards from its rank; top level = height hq
-    if (p - 1 >= 3) {
-        const Idx baseLL = mbq + T.cL(p - 1, hq) + T.cL(p - 2, hq + 1);
-        // u = N: LN = NL - cL(p-1, h) + cL(p, h); blocked [P', L, L, S*] = NL - mainbase + blkbase
-        const Idx dLN = T.mcL(p, h) - T.cL(p - 1, h);
-        const Idx dBL = k.blkbase - k.mainbase;
+// The closure sources of a class in other classes, for both cells in one scan of S'
+// and one of P': of cell p's x=N word [P', N, y, S'] (y = yN, dh(y) = D; sums into
+// clo, values before the pass) and of cell p-1's [P', u, N, S'] (u = yN; sums into
+// clo2, values after cell p).  The sources in the class itself are added by the caller.
+//
+// Cell p's top level is h, cell p-1's hq = h + D, and both words hold the same P' and
+// S', so a scan meets the sources of one cell after those of the other:
+//   S' downwards from height h + D, LL sources (a top-level L turned into R, S*): a
+//     top-level R ends a scan, that is one level lower.  D = 0: both cells' at level h.
+//     D = -1: y = R ends cell p's scan before S'; cell p-1's at hq.  D = 1: cell p-1's at hq = h + 1
+//     up to the R that ends them, from there cell p's at h.
+//   P' upwards from height h, RR sources (a top-level R turned into L, P*): a top-level
+//     L ends a scan, one level lower.  D = 0: both at level h.  D = -1: cell p's at h
+//     up to the L that ends them, from there cell p-1's at h - 1 (u itself flipped is
+//     the caller's).  D = 1: cell p's; u = L ends cell p-1's at once.
+// One scan per cell and side, four in all, was most of a pass's instructions where the
+// index math is the bound (one modulus, 64-bit ranks).  Solves, ms, then and now: n=12 at
+// one modulus 0.57, 0.50; n=15 at 3 1.59, 1.34; n=18 at one 14.6, 13.8; n=21 at one 383.7, 349.5;
+// n=20 at 11 744.7, 732.0; a row of n=23 at one 412.9, 348.6, of n=21 at 13 308.4, 306.3.
+//
+// D = 0: cell p-1's sources [P', N, L, L, S*] and [P*, N, R, R, S'] are NL / NR targets
+// of cell p, rebuilt from old values (NL + LN + blocked; the blocked term only when
+// the blocked input of cell p is valid).  A source's values are added when the next one
+// is found (Late), so the scan runs on while they are on their way.
+template <int KC, int N>
+struct Late {  // N loads in flight per source
+    Vals<KC> v[N];
+    bool have = false;
+};
+
+template <int KC, typename Idx, int D>
+OFP_HD void closures(const Tab<Idx>& T, int W, int p, const Class<Idx>& k, bool read_blk, const Io<KC, Idx>& io,
+                     Vals<KC>& clo, Vals<KC>& clo2, const uint32_t* mod) {
+    constexpr int y = D == 0 ? 0 : (D == -1 ? 1 : 2);
+    const int h = k.h, hq = h + D;
+    // D = 0: cell p's source and cell p-1's three; otherwise one of either cell's
+    Late<KC, D == 0 ? 4 : 1> g;
+    int dst = 0;  // the cell the value in flight belongs to (D != 0): 0 = p, 1 = p-1
+    auto add_late = [&]() {
+        if (!g.have) return;
+        if constexpr (D == 0) {
+            vadd<KC>(clo, g.v[0], mod);
+            vadd<KC>(clo2, g.v[1], mod);
+            vadd<KC>(clo2, g.v[2], mod);
+            if (read_blk) vadd<KC>(clo2, g.v[3], mod);
+        } else {
+            if (dst) vadd<KC>(clo2, g.v[0], mod);
+            else vadd<KC>(clo, g.v[0], mod);
+        }
+    };
+    auto take1 = [&](Idx i, int cell) {
+        add_late();
+        io.lm((uint64_t)i, g.v[0]);
+        dst = cell;
+        g.have = true;
+    };
+    auto take4 = [&](Idx i0, Idx i1, Idx i2, Idx ib) {
+        add_late();
+        if constexpr (D == 0) {
+            io.lm((uint64_t)i0, g.v[0]);
+            io.lm((uint64_t)i1, g.v[1]);
+            io.lm((uint64_t)i2, g.v[2]);
+            if (read_blk) io.lb((uint64_t)ib, g.v[3]);
+        }
+        g.have = true;
+    };
+    // LL
+    {
+        const Idx mL = T.mcL(p, h);
+        // D = 0: [P', L, L, N, S*] and [P', N, L, L, S*] / [P', L, N, L, S*] / blocked [P', L, L, S*]
+        const Idx base = k.mainbase + mL + T.cL(p - 1, h + 1) + (D == 1 ? T.cL(p - 2, h + 2) : Idx(0));  // cell p
+        const Idx base1 = k.mainbase + (D == -1 ? T.mat(p, h) : (D == 1 ? mL : Idx(0))) + T.cL(p - 1, hq) +
+                          T.cL(p - 2, hq + 1);  // cell p-1
         Idx rr = k.sr, s2 = 0;
-        int hh = hq;
+        int hh = hq, lvl = hq;
         for (int pos = p - 3; pos >= 0; --pos) {
             const Z2<Idx> e = ldz(T.q[pos][hh]);
             const Z2<Idx> e2 = ldz(T.q[pos][hh + 2]);
             const bool g0 = rr >= e.zn, g1 = rr >= e.zc;
             rr -= g1 ? e.zc : (g0 ? e.zn : Idx(0));
-            if (g1 && hh == hq) {
-                const Idx i = baseLL + s2 + e2.zn + rr;
-                io.lm((uint64_t)i, t);
-                vadd<KC>(acc, t, mod);
-                if (u == 0) {
-                    io.lm((uint64_t)(Idx)(i + dLN), t);
-                    vadd<KC>(acc, t, mod);
-                    if (read_blk) {
-                        io.lb((uint64_t)(Idx)(i + dBL), t);
-                        vadd<KC>(acc, t, mod);
-                    }
+            if (hh == lvl) {
+                if (g1) {
+                    const Idx q = s2 + e2.zn + rr;  // rank of S*
+                    if constexpr (D == 0)
+                        take4(base + q, base1 + q, base1 + q + (mL - T.cL(p - 1, h)), base1 + q + (k.blkbase - k.mainbase));
+                    else if constexpr (D == -1)
+                        take1(base1 + q, 1);
+                    else
+                        take1((lvl == hq ? base1 : base) + q, lvl == hq);
+                } else if (g0) {
+                    if (D != 1 || lvl == h) break;
+                    lvl = h;
                 }
             }
-            if (g0 && !g1 && hh == hq) break;
             s2 += g1 ? e2.zc : (g0 ? e2.zn : Idx(0));
             hh += g1 ? 1 : (g0 ? -1 : 0);
         }
     }
-    // RR over P' (positions p+1 and up); an L at the top level ends it.  u = L
-    // ends it at once (its own position is the top level), u = R raises the
-    // depth of everything above it.
-    if (u == 2) return;
+    // RR.  vm + (the entry of the L at the flip) + u2 is P*'s rank contribution in the main
+    // numbering, vb + ... + b2 in the blocked one (D = 0): the unscanned part, the flip and the
+    // scanned part two levels higher.
     {
-        // candidate main index = ub + (L contribution at the flip) + u2:
-        //   ub: main contributions of the unscanned part of P', plus u at its
-        //       height in P'* (h + 2), the two R's of the window and S';
-        //   u2: main contributions of the scanned part of P' two levels higher.
-        // The blocked index of [P'*, R, R, S'] (needed when u = N) differs from
-        // the main index of [P'*, N, R, R, S'] by the blocked-minus-main
-        // contributions of P'*: db (unscanned) + dl (flip) + d2 (scanned, +2).
-        const int hs = h + 2;  // height entering position p in P'*
-        Idx ub = k.mainbase + mcontrib(T, p, u, hs) + T.at(p - 1, hq + 2) + T.at(p - 2, hq + 1) + k.sr;
-        Idx u2 = 0, db = k.blkbase - k.mainbase, d2 = 0;
-        const Idx dRN = T.mat(p, hs) - T.at(p - 1, hs);  // u = N: RN - NR in P'*
-        int Ha = h;  // height below the scanned position (after u and the window)
+        const int hs = h + 2;  // height entering position p in P*'s words
+        const Idx in0 = T.mat(p, hs) + T.at(p - 1, h + 1) + contrib(T, p - 2, y, h) + k.sr;  // R, R, y, S'
+        // cell p-1: [u, R, R, S'] at p, p-1, p-2 and the blocked [R, R, S'] (u = N)
+        const Idx in1 = D == 1 ? Idx(0)
+                               : Idx((D == -1 ? T.mat(p, hs) : Idx(0)) + T.at(p - 1, hq + 2) + T.at(p - 2, hq + 1) + k.sr);
+        const Idx dRN = T.mat(p, hs) - T.at(p - 1, hs);  // u = N: RN - NR
+        Idx vm = k.mainbase, u2 = 0, vb = k.blkbase, b2 = 0;
+        int Ha = h, lvl = h;
         uint64_t w = k.word >> (2 * p);
         for (int mp = p + 1; mp <= W - 1; ++mp) {
             const uint32_t v = (uint32_t)w & 3u;
             w >>= 2;
             const bool isR = v == 1, isL = v == 2;
             const int H = Ha + (isR ? 1 : (isL ? -1 : 0));
-            const Quad<Idx> e0 = ldq(T.q[mp - 1][H]);
-            const Quad<Idx> e2 = ldq(T.q[mp - 1][H + 2]);
-            // remove this position's contributions from the unscanned sums
-            ub -= isL ? e0.mc : (isR ? e0.mn : Idx(0));
-            db -= isL ? (e0.zc - e0.mc) : (isR ? (e0.zn - e0.mn) : Idx(0));
-            const bool atTop = Ha == hq;  // top level of the x'=N word's prefix
-            if (isR && atTop) {
-                const Idx i = ub + e0.mc + u2;
-                io.lm((uint64_t)i, t);
-                vadd<KC>(acc, t, mod);
-                if (u == 0) {
-                    io.lm((uint64_t)(Idx)(i + dRN), t);
-                    vadd<KC>(acc, t, mod);
-                    if (read_blk) {
-                        io.lb((uint64_t)(Idx)(i + db + (e0.zc - e0.mc) + d2), t);
-                        vadd<KC>(acc, t, mod);
-                    }
+            Quad<Idx> e0{}, e2{};
+            if constexpr (D == 0) {
+                e0 = ldq(T.q[mp - 1][H]);
+                e2 = ldq(T.q[mp - 1][H + 2]);
+                vb -= isL ? e0.zc : (isR ? e0.zn : Idx(0));
+            } else {
+                const Z2<Idx> m0 = cell::ldm(T.q[mp - 1][H]), m2 = cell::ldm(T.q[mp - 1][H + 2]);
+                e0.mn = m0.zn, e0.mc = m0.zc, e2.mn = m2.zn, e2.mc = m2.zc;
+            }
+            vm -= isL ? e0.mc : (isR ? e0.mn : Idx(0));
+            if (Ha == lvl) {
+                if (isR) {
+                    const Idx q = vm + e0.mc + u2;
+                    if constexpr (D == 0)
+                        take4(q + in0, q + in1, q + in1 + dRN, vb + e0.zc + b2 + in1);
+                    else if constexpr (D == -1)
+                        take1(q + (lvl == h ? in0 : in1), lvl != h);
+                    else
+                        take1(q + in0, 0);
+                } else if (isL) {
+                    if (D != -1 || lvl != h) break;
+                    lvl = hq;
                 }
             }
-            if (isL && atTop) break;
             u2 += isL ? e2.mc : (isR ? e2.mn : Idx(0));
-            d2 += isL ? (e2.zc - e2.mc) : (isR ? (e2.zn - e2.mn) : Idx(0));
+            if constexpr (D == 0) b2 += isL ? e2.zc : (isR ? e2.zn : Idx(0));
             Ha = H;
         }
     }
+    add_late();
 }
 
 // The pass over one class of window change D.  GF = 0: the class's words are
@@ -398,34 +450,16 @@ OFP_HD void pair_body(const PairLaunch& a, const Tab<Idx>& T, const Class<Idx>& 
         pb[i] = h1 >= 0;
         ib[i] = (uint64_t)(Idx)(k.blkbase + contrib(T, p - 1, x, h) + contrib(T, p - 2, y, h1 < 0 ? 0 : h1) + k.sr);
     }
-    // closure sums read from memory: cell p's x=N word (sources before cell p)
-    // and cell p-1's x'=N word (sources in other classes, rebuilt as after cell p)
+    // closure sums read from other classes' words: cell p's x=N word's (sources before
+    // cell p) and cell p-1's x'=N word's (rebuilt as after cell p)
     Vals<KC> clo, clo2;
     vzero<KC>(clo);
     vzero<KC>(clo2);
-    auto gather_p = [&]() {
-        if constexpr (yN >= 0) {
-            if (pb[S::b(0, yN)]) {
-                cell::Gather<KC, cell::kAoS> g;
-                g.init();
-                const cell::Direct<KC, cell::kAoS, Idx> old{const_cast<uint32_t*>(io.mi),
-                                                            const_cast<uint32_t*>(io.bi), io.K, io.off};
-                const Idx srp = contrib(T, p - 2, yN, h) + k.sr;  // rank of S = (y, S') entered at h
-                cell::gather_closures<KC, Idx, cell::kAoS>(T, W, p, h, k.mainbase, srp, k.word, old, g, mod);
-                g.finish(old, mod);
-                clo = g.acc;
-            }
-        }
+    // both words are there in every class: h >= 0, and h + D >= 0 where S' begins
+    auto gather = [&]() {
+        if constexpr (yN >= 0) closures<KC, Idx, D>(T, W, p, k, a.read_blk != 0, io, clo, clo2, mod);
     };
-    auto gather_p1 = [&]() {
-        if constexpr (yN >= 0) {
-            if (pb[S::b(yN, 0)]) closures_after<KC, Idx>(T, W, p, k, yN, a.read_blk != 0, io, clo2, mod);
-        }
-    };
-    if constexpr (GF == 1) {
-        gather_p();
-        gather_p1();
-    }
+    if constexpr (GF == 1) gather();
     Vals<KC> m[S::NM > 0 ? S::NM : 1];
 #pragma unroll
     for (int i = 0; i < S::NM; ++i) {
@@ -438,6 +472,7 @@ OFP_HD void pair_body(const PairLaunch& a, const Tab<Idx>& T, const Class<Idx>& 
         if (pb[i] && a.read_blk) io.lb(ib[i], bl[i]);
         else vzero<KC>(bl[i]);
     }
+    if constexpr (GF == 0) gather();
 
     // Cell-by-cell, the orbits whose blocked word is x=R or x=L first and the x=N
     // orbit (whose blocked output is the closure sum) last, so that the closure
@@ -472,7 +507,11 @@ OFP_HD void pair_body(const PairLaunch& a, const Tab<Idx>& T, const Class<Idx>& 
         constexpr int iNN = S::m(0, 0, yN), iLR = S::m(2, 1, yN);
         vadd<KC>(m[iLR], m[iNN], mod);
         vadd<KC>(m[iNN], bl[i], mod);
-        if constexpr (GF == 0) gather_p();
+        // sources in the class (cell p keeps both): RL = [P', R, L, y, S'], and with y = L
+        // the LL source with y itself turned into R, [P', L, L, R, S']
+        constexpr int iRL = S::m(1, 2, yN);
+        if (pm[iRL]) vadd<KC>(clo, m[iRL], mod);
+        if constexpr (yN == 2) vadd<KC>(clo, m[S::m(2, 2, 1)], mod);
         bl[i] = clo;  // blocked output: the closure sum
     }
 
@@ -526,7 +565,6 @@ OFP_HD void pair_body(const PairLaunch& a, const Tab<Idx>& T, const Class<Idx>& 
                 constexpr int iLRR = S::m(2, 1, 1);
                 if (pm[iLRR]) vadd<KC>(clo2, m[iLRR], mod);
             }
-            if constexpr (GF == 0) gather_p1();
         }
         vadd<KC>(m[iLR], m[iNN], mod);
         vadd<KC>(m[iNN], bl[i], mod);
