@@ -533,16 +533,16 @@ bool pair_ready(const ofp_ctx* c, const Sweep& s) { return pairs_apply(c, s.n) &
 
 // Cells p_hi..p_lo of s, walking down from p_hi: where bit p of the context's
 // pair mask is set and p-1 >= p_lo, cells p and p-1 run as one pair pass (in
-// place, one launch per window height change d, the classes that read other
-// classes -- d = -1, 0, 1 -- first), otherwise cell p runs alone with the
+// place, one launch per window height change d, or one for those whose classes
+// read other classes -- d = -1, 0, 1 --, which go first), otherwise cell p runs alone with the
 // per-cell kernel.  The first cell reads the blocked input iff first_reads_blk.
 // With cell_ev, events bracket each step: a pair's first cell slot (slot
 // p_hi - p, kind 2) gets its time and the second an empty interval (kind 3).
-// The library's default pairing: every pair except the one over cells 4 and 3,
-// which runs as two launches (n=22: 125 against 60 + 66 ms at 14 moduli, 27.4
-// against 12.8 + 13.3 ms at one modulus; the other passes are 1.2-1.5x faster
-// than their two cells).
-uint32_t default_pair_mask(int) { return ~((1u << 4) | (1u << 3)); }
+// The library's default pairing: every pair except cells 3 and 2 (n=21 at 13 moduli
+// 50.9 ms, with cell 1 alone 75.3; cell 3 alone and 2, 1 65.3) and, from 2 to 7 moduli, cells 4
+// and 3 (n=20 at 4 6.2 against 2.7 + 2.9 ms; at 11 13.4 against 6.9 + 7.2, n=18 at one 0.28
+// against 0.19 + 0.19).  The other passes are 1.05-1.9x faster than their two cells.
+uint32_t default_pair_mask(int kc) { return ~((1u << 3) | (kc > 1 && kc < 8 ? 1u << 4 : 0u)); }
 // Group sweeps (4 moduli, n=27 windows over three streams): pair passes over
 // every pair of cells from 7 up; cells 6..1 one per launch, where the pair
 // pass over a group is no faster than its two cells (6, 5: 781 against 780 ms
@@ -616,6 +616,21 @@ ofp_status enqueue_pair_whole(ofp_ctx* c, Sweep& s, int p, bool reads_blk, int c
     return OFP_OK;
 }
 
+// Chunks of d = 0's classes a workgroup takes at a time where a pass's readers (d = -1,
+// 0, 1) run as one launch (pair_readers_kernel), 0 where each d has its own.  Below the
+// window few positions are left at low cells, so the words of one P' lie side by side and three
+// launches move every line three times; high up a P' has many words of each d, lines are not
+// shared, and pieces of one P' would be too few and too uneven.  ms of a pass, three
+// launches and one: n=21 at 13 moduli cells 9, 8 25.9, 24.5; 7, 6 30.0, 27.2; 5, 4
+// 41.5, 35.9; n=20 at 11 10, 9 7.27, 7.04; 12, 11 6.94, 7.52; 16, 15 6.88, 19.9; n=20 at 4 6, 5
+// 4.74, 3.79.  One modulus shares lines too but is bound by its index math, and there
+// the shorter pieces cost as much as they save: n=21 5, 4 7.88, 7.20; 7, 6 4.29, 4.24; 9, 8
+// 2.57, 3.12.
+int reader_pieces(int W, int p, int kc) {
+    if (p >= W - 1) return 0;  // no P' to cut at
+    return kc == 1 ? (p <= 5 ? 2 : 0) : (p <= 10 ? 1 : 0);
+}
+
 // One pair pass over cells p and p-1 (cap > 0: over the classes at heights <= cap).
 ofp_status enqueue_pair(ofp_ctx* c, Sweep& s, int p, bool reads_blk, int cap, int* launches) {
     if (whole_ready(c, s)) return enqueue_pair_whole(c, s, p, reads_blk, cap, launches);
@@ -646,11 +661,14 @@ ofp_status enqueue_pair(ofp_ctx* c, Sweep& s, int p, bool reads_blk, int cap, in
             }
             return OFP_OK;
         };
+        const int pieces = pair_class_count(W, p, 0, cap) ? reader_pieces(W, p, kc) : 0;
         for (int di = 0; di < 5; ++di) {
             const int d = kOrder[di];
-            if (di == 3)
+            const bool all = pieces && d == 0;  // the launch of all three readers, on s.stream
+            if (pieces && di < 3 && !all) continue;
+            if (di == 3 && !pieces)
                 if (ofp_status f = join()) return f;
-            if (di == 0 || di == 3)
+            if ((di == 0 && !pieces) || di == 3)
                 if (ofp_status f = fork()) return f;
             const uint64_t cnt = pair_class_count(W, p, d, cap);
             if (!cnt) continue;
@@ -661,6 +679,12 @@ ofp_status enqueue_pair(ofp_ctx* c, Sweep& s, int p, bool reads_blk, int cap, in
             a.blk_out = s.blk;
             a.dp = wide ? c->dp64 : c->dp32;
             a.ct = static_cast<const char*>(wide ? c->ct64 : c->ct32) + tb * (size_t)((cap * kMaxW + p) * 7 + d + 3);
+            if (all) {
+                a.ct = static_cast<const char*>(wide ? c->ct64 : c->ct32) + tb * (size_t)(cap * kMaxW + p) * 7;
+                a.ct_bytes = (uint32_t)tb;
+                for (int side = 0; side < 2; ++side) a.sides[side] = pair_class_count(W, p, 2 * side - 1, cap);
+                a.group = pieces;
+            }
             a.classes = cnt;
             a.W = W;
             a.p = p;
@@ -673,8 +697,10 @@ ofp_status enqueue_pair(ofp_ctx* c, Sweep& s, int p, bool reads_blk, int cap, in
             for (int jj = 0; jj < kc; ++jj) a.mod[jj] = s.mods[off + jj];
             a.xcd_shift = piece_shift(c->xcd_shift, cnt, c->threads);
             a.variant = c->pair_variant;
+            if (all) a.xcd_shift = piece_shift(c->xcd_shift, cnt, c->threads * pieces);
             hipStream_t ls = !par ? s.stream : (d == -1 || d == -2) ? s.par[0] : (d == 1 ? s.par[1] : s.stream);
-            hipError_t e = launch_pair(a, wide, c->threads, grid_blocks(c, cnt), ls);
+            hipError_t e = all ? launch_pair_readers(a, wide, c->threads, grid_blocks(c, cnt), ls)
+                               : launch_pair(a, wide, c->threads, grid_blocks(c, cnt), ls);
             if (e != hipSuccess) return hip_fail(c, e, "pair pass launch");
             if (launches) ++*launches;
         }

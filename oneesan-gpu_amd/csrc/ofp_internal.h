@@ -115,6 +115,7 @@ size_t class_table_bytes(bool wide);
 // Classes of (p, d) in a row of width W (cap > 0: those at heights <= cap).
 uint64_t pair_class_count(int W, int p, int d, int cap);
 // One pair-pass launch (a.kc in 1..16 moduli).
+hipError_t launch_pair_readers(const pair::PairLaunch& a, bool wide, int threads, int blocks, hipStream_t s);
 hipError_t launch_pair(const pair::PairLaunch& a, bool wide_index, int threads, int blocks, hipStream_t s);
 // A pair pass from main_in / blk_in to main_out / blk_out in one launch (32-bit ranks,
 // at most kWholeKC moduli; ofp_pair_whole.hip).

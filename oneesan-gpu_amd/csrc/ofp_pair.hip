@@ -1,5 +1,6 @@
 // ofp_pair.hip -- the pair pass: cells p and p-1 of a row applied in place,
-// one launch per window height change d (body and design in ofp_pair_impl.h).
+// one launch per window height change d, or one for d = -1, 0 and 1 (body and design
+// in ofp_pair_impl.h; which one: reader_pieces in ofp_api.hip).
 //
 // Each thread takes one class (P', d, S'), decoded from its class number with
 // the class completion table of (p, d) and the height table, both in LDS; the
@@ -40,6 +41,56 @@ __global__ __launch_bounds__(256, MB) void pair_kernel(pair::PairLaunch a) {
             const pair::Class<Idx> k = Capped ? pair::decode_class_capped<Idx>(T, ctab, a.W, a.p, D, c)
                                               : pair::decode_class<Idx>(T, ctab, a.W, a.p, c);
             pair::pair_body<KC, Idx, D, GF>(a, T, k, io);
+        }
+    }
+}
+
+// The classes of d = -1, 0 and 1 in one launch, a piece of the prefixes P' at a time: a
+// workgroup takes a.group chunks of d = 0's classes and, with them, the d = -1 and 1
+// classes of the same P' (from the first P' of its chunks to that of the next ones).
+template <int KC, typename Idx, bool Capped>
+__global__ __launch_bounds__(256, 2) void pair_readers_kernel(pair::PairLaunch a) {
+    constexpr int C = LdsCols<Idx>::value;
+    __shared__ Quad<Idx> tab[kLdsRows][C];
+    __shared__ Pair<Idx> ctab[kLdsRows][C];
+    __shared__ uint64_t at[2], word[2];  // the piece's ends: classes of one d; P' (all ones: past the last)
+    load_table<C, kDpCols>(&tab[0][0], (const Quad<Idx>*)a.dp, a.W);
+    const Tab<Idx> T{tab};
+    const pair::Io<KC, Idx> io{a.main_in, a.blk_in, a.main_out, a.blk_out, a.K, a.off};
+    const uint64_t piece = (uint64_t)blockDim.x * (uint32_t)a.group;
+    const Sched sc(a.classes, (uint32_t)piece, gridDim.x, blockIdx.x, a.xcd_shift);
+    auto table = [&](int d) {
+        __syncthreads();  // the last one's readers
+        load_table<C, C>(&ctab[0][0], (const Pair<Idx>*)((const char*)a.ct + (size_t)(d + 3) * a.ct_bytes), a.W);
+        __syncthreads();
+    };
+    auto decode = [&](int d, uint64_t c) {
+        return Capped ? pair::decode_class_capped<Idx>(T, ctab, a.W, a.p, d, c)
+                      : pair::decode_class<Idx>(T, ctab, a.W, a.p, c);
+    };
+    for (uint64_t t = sc.slot; t < sc.count; t += sc.nx) {
+        const uint64_t lo = sc.chunk(t) * piece, hi = lo + piece < a.classes ? lo + piece : a.classes;
+        if (lo >= a.classes) continue;  // the whole workgroup
+        table(0);
+        if (threadIdx.x < 2) {
+            const uint64_t c = threadIdx.x ? hi : lo;
+            word[threadIdx.x] = c < a.classes ? pair::decode_class<Idx>(T, ctab, a.W, a.p, c).word : ~0ull;
+        }
+        for (uint64_t c = lo + threadIdx.x; c < hi; c += blockDim.x)
+            pair::pair_body<KC, Idx, 0, 0>(a, T, decode(0, c), io);
+        for (int side = 0; side < 2; ++side) {
+            table(2 * side - 1);
+            if (threadIdx.x < 2)
+                at[threadIdx.x] = threadIdx.x == 0 && lo == 0 ? 0
+                                  : word[threadIdx.x] == ~0ull
+                                      ? a.sides[side]
+                                      : (uint64_t)pair::classes_before<Idx>(ctab, a.W, a.p, word[threadIdx.x]);
+            __syncthreads();
+            const uint64_t b = at[0], e = at[1];
+            for (uint64_t c = b + threadIdx.x; c < e; c += blockDim.x) {
+                if (side == 0) pair::pair_body<KC, Idx, -1, 0>(a, T, decode(-1, c), io);
+                else pair::pair_body<KC, Idx, 1, 0>(a, T, decode(1, c), io);
+            }
         }
     }
 }
@@ -148,6 +199,28 @@ uint64_t pair_class_count(int W, int p, int d, int cap) {
     for (int h = std::max(0, -d); h + std::max(0, d) < kDpCols; ++h)
         n += words.up[cap][W - 1 - p][h] * words.down[cap][p - 2][h + d];
     return n;
+}
+
+hipError_t launch_pair_readers(const pair::PairLaunch& a, bool wide, int threads, int blocks, hipStream_t s) {
+    if (a.p < 2 || a.p > a.W - 1 || a.kc < 1 || a.off + a.kc > a.K || a.cap < 0 || a.cap > kPairCaps || !a.classes ||
+        a.group < 1 || threads <= 0 || threads > 256 || (threads & 63) || blocks <= 0 || (blocks & 7))
+        return hipErrorInvalidValue;
+#define OFP_R(n, I)                                                                                                \
+    if (a.cap > 0) hipLaunchKernelGGL((pair_readers_kernel<n, I, true>), dim3(blocks), dim3(threads), 0, s, a);     \
+    else hipLaunchKernelGGL((pair_readers_kernel<n, I, false>), dim3(blocks), dim3(threads), 0, s, a);
+    switch (a.kc) {
+#define OFP_KC(n)                                      \
+    case n:                                            \
+        if (wide) { OFP_R(n, uint64_t) }               \
+        else { OFP_R(n, uint32_t) }                    \
+        break;
+        OFP_KC(1) OFP_KC(2) OFP_KC(3) OFP_KC(4) OFP_KC(5) OFP_KC(6) OFP_KC(7) OFP_KC(8)
+        OFP_KC(9) OFP_KC(10) OFP_KC(11) OFP_KC(12) OFP_KC(13) OFP_KC(14) OFP_KC(15) OFP_KC(16)
+#undef OFP_KC
+#undef OFP_R
+        default: return hipErrorInvalidValue;
+    }
+    return hipGetLastError();
 }
 
 hipError_t launch_pair(const pair::PairLaunch& a, bool wide, int threads, int blocks, hipStream_t s) {

@@ -150,6 +150,10 @@ struct PairLaunch {
     // workgroup and class table (ct + (d + 3) * ct_bytes) of each
     uint32_t count[7], block[8];
     uint32_t ct_bytes;
+    // one launch over d = -1, 0 and 1 (launch_pair_readers): ct as above, classes those of
+    // d = 0, sides those of -1 and 1, group: chunks of d = 0 a workgroup takes at a time
+    uint64_t sides[2];
+    int group;
     uint32_t mod[kMaxKC];
 };
 
@@ -189,6 +193,20 @@ OFP_HD Class<Idx> decode_class(const Tab<Idx>& T, const cell::Pair<Idx> (*ct)[ce
     k.word = word << (2 * p);
     k.h = h;
     return k;
+}
+
+// Classes of ct's (p, d) whose P' comes before the P' of `word` (as in Class).
+template <typename Idx>
+OFP_HD Idx classes_before(const cell::Pair<Idx> (*ct)[cell::LdsCols<Idx>::value], int W, int p, uint64_t word) {
+    Idx n = 0;
+    int h = 1;
+    for (int m = W - 1; m >= p + 1; --m) {
+        const int v = (int)(word >> (2 * (m - 1))) & 3;
+        const cell::Pair<Idx> g = ct[m][h];
+        n += pick(v, g.n, g.c);
+        h += dh(v);
+    }
+    return n;
 }
 
 // Decode class number c among the classes of (p, d) whose P' and S' stay at heights
