@@ -33,10 +33,11 @@ struct Sweep {
     uint32_t* main = nullptr;
     uint32_t* blk = nullptr;
     size_t main_cap = 0, blk_cap = 0;  // bytes allocated
-    // small states: a second pair of arrays, as large, that a pair pass goes to (and the
-    // two pairs change places); null: none
+    // small states: a second pair of arrays that a pair pass goes to (and the two pairs
+    // change places); null: none
     uint32_t* main2 = nullptr;
     uint32_t* blk2 = nullptr;
+    size_t main2_cap = 0, blk2_cap = 0;
     bool whole = false;  // both pairs started from one state (init_state)
     uint32_t* mods_dev = nullptr;
     int mods_cap = 0;
@@ -225,6 +226,19 @@ void sweep_free(Sweep& s, void* p) {
     else (void)hipFree(p);
 }
 
+void free_second(Sweep& s) {
+    sweep_free(s, s.main2);
+    sweep_free(s, s.blk2);
+    s.main2 = s.blk2 = nullptr;
+    s.main2_cap = s.blk2_cap = 0;
+}
+void swap_pairs(Sweep& s) {
+    std::swap(s.main, s.main2);
+    std::swap(s.blk, s.blk2);
+    std::swap(s.main_cap, s.main2_cap);
+    std::swap(s.blk_cap, s.blk2_cap);
+}
+
 void free_sweep(Sweep& s) {
     drop_graph(s);
     for (hipEvent_t e : s.seg_ev) (void)hipEventDestroy(e);
@@ -246,7 +260,7 @@ void free_sweep(Sweep& s) {
     sweep_free(s, s.gscratch);
     s.main = s.blk = s.main2 = s.blk2 = s.mods_dev = s.gscratch = nullptr;
     s.acc = nullptr;
-    s.main_cap = s.blk_cap = s.gscratch_cap = 0;
+    s.main_cap = s.blk_cap = s.main2_cap = s.blk2_cap = s.gscratch_cap = 0;
     s.mods_cap = 0;
     s.layout = -1;
 }
@@ -357,14 +371,14 @@ ofp_status ensure_state(ofp_ctx* c, Sweep& s, int n, const uint32_t* moduli, int
     size_t mb = padded_states(nm) * (size_t)Kp * sizeof(uint32_t);
     size_t bb = padded_states(nb ? nb : 1) * (size_t)Kp * sizeof(uint32_t);
     OFP_HIP(c, hipSetDevice(c->device), "hipSetDevice");
+    if (s.main2_cap > s.main_cap) swap_pairs(s);  // the larger pair holds the state
     if (mb > s.main_cap || bb > s.blk_cap) {
         drop_graph(s);
         sweep_free(s, s.main);
         sweep_free(s, s.blk);
-        sweep_free(s, s.main2);
-        sweep_free(s, s.blk2);
-        s.main = s.blk = s.main2 = s.blk2 = nullptr;
+        s.main = s.blk = nullptr;
         s.main_cap = s.blk_cap = 0;
+        free_second(s);
         release_window(c);
         size_t fr = 0, tot = 0;
         OFP_HIP(c, hipMemGetInfo(&fr, &tot), "hipMemGetInfo");
@@ -377,10 +391,18 @@ ofp_status ensure_state(ofp_ctx* c, Sweep& s, int n, const uint32_t* moduli, int
         s.blk_cap = bb;
     }
     s.whole = false;
-    if (whole_size(c, n, k)) {  // without the room, as above these sizes
-        if (!s.main2 && sweep_alloc(s, (void**)&s.main2, s.main_cap) != hipSuccess) s.main2 = nullptr;
-        if (!s.blk2 && sweep_alloc(s, (void**)&s.blk2, s.blk_cap) != hipSuccess) s.blk2 = nullptr;
-        (void)hipGetLastError();
+    // the second pair: of this state's size, however large the first one still is from an
+    // earlier solve; without the room the state is swept as above these sizes
+    if (whole_size(c, n, k) && (mb > s.main2_cap || bb > s.blk2_cap)) {
+        free_second(s);
+        if (sweep_alloc(s, (void**)&s.main2, mb) != hipSuccess) s.main2 = nullptr;
+        if (s.main2 && sweep_alloc(s, (void**)&s.blk2, bb) != hipSuccess) s.blk2 = nullptr;
+        s.main2_cap = mb;
+        s.blk2_cap = bb;
+        if (!s.blk2) {
+            (void)hipGetLastError();
+            free_second(s);
+        }
     }
     if (s.mods_cap < k) {
         sweep_free(s, s.mods_dev);
@@ -611,8 +633,7 @@ ofp_status enqueue_pair_whole(ofp_ctx* c, Sweep& s, int p, bool reads_blk, int c
         if (e != hipSuccess) return hip_fail(c, e, "pair pass launch");
         if (launches) ++*launches;
     }
-    std::swap(s.main, s.main2);
-    std::swap(s.blk, s.blk2);
+    swap_pairs(s);
     return OFP_OK;
 }
 
@@ -1329,7 +1350,7 @@ ofp_status ofp_plan(ofp_ctx* c, int n, int k, ofp_plan_info* out) {
     OFP_HIP(c, hipSetDevice(c->device), "hipSetDevice");
     OFP_HIP(c, hipMemGetInfo(&fr, &tot), "hipMemGetInfo");
     // memory already held by this context's own state can be reused
-    out->free_bytes = fr + c->st.main_cap + c->st.blk_cap;
+    out->free_bytes = fr + c->st.main_cap + c->st.blk_cap + c->st.main2_cap + c->st.blk2_cap;
     out->fits = out->state_bytes + c->reserve <= out->free_bytes;
     return OFP_OK;
 }
@@ -1462,7 +1483,7 @@ ofp_status ofp_solve(ofp_ctx* c, int n, const uint32_t* moduli, int k, uint32_t*
     size_t fr = 0, tot = 0;
     OFP_HIP(c, hipSetDevice(c->device), "hipSetDevice");
     OFP_HIP(c, hipMemGetInfo(&fr, &tot), "hipMemGetInfo");
-    const uint64_t avail = fr + c->st.main_cap + c->st.blk_cap + c->win_bytes + c->stage_bytes;
+    const uint64_t avail = fr + c->st.main_cap + c->st.blk_cap + c->st.main2_cap + c->st.blk2_cap + c->win_bytes + c->stage_bytes;
     int g = c->max_batch > 0 ? std::min(k, c->max_batch) : k;
     while (g > 1 && state_bytes(c->layout, n, g) + c->reserve > avail) --g;
     if (state_bytes(c->layout, n, g) + c->reserve > avail)
@@ -1525,6 +1546,8 @@ ofp_status ofp_solve_static(ofp_ctx* c, int n, const uint32_t* moduli, int k, ui
     const bool two = whole_size(c, n, k) && 2 * (mb + bb) <= kStaticStateBytes;  // room for the second pair
     s.main2 = two ? s.blk + bb / sizeof(uint32_t) : nullptr;
     s.blk2 = two ? s.main2 + mb / sizeof(uint32_t) : nullptr;
+    s.main2_cap = two ? mb : 0;
+    s.blk2_cap = two ? bb : 0;
     s.mods_dev = nullptr;  // the start word takes the moduli by value
     s.acc = c->static_acc;
     s.mods.assign(moduli, moduli + k);
@@ -1542,6 +1565,7 @@ ofp_status ofp_solve_static(ofp_ctx* c, int n, const uint32_t* moduli, int k, ui
     if (st) return st;
     st = read_main(c, s, 0, residues_out, k);
     s.main = s.blk = s.main2 = s.blk2 = nullptr;
+    s.main2_cap = s.blk2_cap = 0;
     return st;
 }
 

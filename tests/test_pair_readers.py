@@ -38,3 +38,17 @@ def test_every_cell_paired(bits, n, k, oracle):
         assert ctx.solve(n, MODS[:k])[0] == [oracle.solve(n, m) for m in MODS[:k]]
         ctx.set_height_caps(False)  # all rows, whole
         assert ctx.solve(n, MODS[:k])[0] == [oracle.solve(n, m) for m in MODS[:k]]
+
+
+@pytest.mark.gpu
+def test_second_pair_of_arrays_has_the_small_states_size(oracle):
+    """A small solve on a context that holds a large state takes a second pair of arrays of
+    its own size, and the large state's arrays serve the next large solve."""
+    import ofp
+    with ofp.Context() as ctx, ofp.Context() as other:  # the other one holds no state
+        big = ctx.solve(18, MODS[:8])[0]
+        free = other.plan(12, 1).free_bytes
+        for n in (12, 11, 12):
+            assert ctx.solve(n, MODS[:1])[0] == [oracle.solve(n, MODS[0])]
+        assert free - other.plan(12, 1).free_bytes < 64 << 20
+        assert ctx.solve(18, MODS[:8])[0] == big
