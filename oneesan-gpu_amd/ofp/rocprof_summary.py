@@ -56,17 +56,27 @@ def _short(name: str) -> str:
 
 
 def _kc(name: str) -> int | None:
-    m = re.search(r"(?:cell_(?:capped_|sorted_)?|pair_)kernel<(\d+)", name)
+    m = re.search(r"(?:cell_(?:capped_|sorted_)?|pair_(?:readers_)?)kernel<(\d+)", name)
     return int(m.group(1)) if m else None
 
 
 _PAIR_ORDER = {-1: 0, 0: 1, 1: 2, -2: 3, 2: 4, -3: 5, 3: 6}
 
 
-def _pair_d(name: str) -> int | None:
-    """Height change d of a pair_kernel launch (its third template argument)."""
+READERS = (-1, 0, 1)  # the d's of a pair_readers_kernel launch
+
+
+def _pair_d(name: str) -> int | tuple | None:
+    """Height change d of a pair_kernel launch (its third template argument), the three
+    of a pair_readers_kernel launch."""
+    if "pair_readers_kernel<" in name:
+        return READERS
     m = re.search(r"pair_kernel<\d+,\s*[^,]+,\s*(-?\d+)", name)
     return int(m.group(1)) if m else None
+
+
+def _ds(d) -> set:
+    return set(d) if isinstance(d, tuple) else {d}
 
 
 def _steps(seq):
@@ -83,13 +93,13 @@ def _steps(seq):
             out.append([t0, t1, capped, 1])
             seen = None
             continue
-        if seen is not None and d not in seen:
+        if seen is not None and not _ds(d) & seen:
             out[-1][1] = max(out[-1][1], t1)
             out[-1][2] = out[-1][2] or capped
-            seen.add(d)
+            seen |= _ds(d)
         else:
             out.append([t0, t1, capped, 2])
-            seen = {d}
+            seen = _ds(d)
     return [(a, (b - a) / 1e6, c, n) for a, b, c, n in out]
 
 
@@ -107,10 +117,10 @@ def _step_rows(seq, cells):
 
 def kernel_family(name: str) -> str | None:
     """'cell_sorted_kernel<14>', 'pair_kernel<14>' etc. for a cell or pair kernel's
-    full name (index width, window change and other template arguments dropped),
-    None for any other kernel."""
-    m = re.search(r"((?:cell_(?:capped_|sorted_|shard_)?|pair_)kernel)<(\d+)", name)
-    return f"{m.group(1)}<{m.group(2)}>" if m else None
+    full name (index width, window change and other template arguments dropped; a pass's
+    one launch over its readers counts as pair_kernel), None for any other kernel."""
+    m = re.search(r"((?:cell_(?:capped_|sorted_|shard_)?|pair_(?:readers_)?)kernel)<(\d+)", name)
+    return f"{m.group(1).replace('readers_', '')}<{m.group(2)}>" if m else None
 
 
 MAX_ROWS = None  # only the first rows of each moduli count (--rows); None = all
@@ -229,12 +239,12 @@ def valu(path: str, cells: int, cus: int, xcds: int, words: int | None) -> None:
             if pd is None:
                 steps.append([[d], capped, 1])
                 seen = None
-            elif seen is not None and pd not in seen:
+            elif seen is not None and not _ds(pd) & seen:
                 steps[-1][0].append(d)
-                seen.add(pd)
+                seen |= _ds(pd)
             else:
                 steps.append([[d], capped, 2])
-                seen = {pd}
+                seen = _ds(pd)
         rows, cur, n = [], [], 0
         for st in steps:
             cur.append(st)
@@ -309,7 +319,7 @@ def dram(path: str) -> None:
               f"{(o['read'] + o['write']) / 1e9:10.3f}")
 
 
-_PAIR_D = re.compile(r"pair_kernel<(\d+), [^,]+, (-?\d+),")
+_PAIR_D = re.compile(r"pair_(?:kernel<(\d+), [^,]+, (-?\d+),|readers_kernel<(\d+))")
 _ORDER = (-1, 0, 1, -2, 2)
 
 
@@ -339,7 +349,8 @@ def launches(path: str) -> None:
         fam = kernel_family(e["kernel"])
         m = _PAIR_D.search(e["kernel"])
         if m:
-            kc, dd = int(m.group(1)), int(m.group(2))
+            readers = m.group(3) is not None
+            kc, dd = int(m.group(3) or m.group(1)), -1 if readers else int(m.group(2))
             i = _ORDER.index(dd) if dd in _ORDER else 99
             if kc != prev_kc or i <= prev_i:
                 close(pas)
@@ -349,7 +360,7 @@ def launches(path: str) -> None:
             pas["rd"] += rd
             pas["wr"] += wr
             pas["n"] += 1
-            dtxt = str(dd)
+            dtxt = "r" if readers else str(dd)
         else:
             close(pas)
             pas, prev_kc, prev_i = None, None, 99
