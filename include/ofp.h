@@ -155,19 +155,21 @@ ofp_status ofp_time_cells(ofp_ctx* ctx, float* ms_out, int* kind_out, int capaci
  * of the context's own solves (ofp_solve, ofp_prepare + ofp_row_sweep,
  * ofp_apply_cells, ofp_time_cells).  A pair pass applies cells p and p-1 in
  * place, in up to five launches (one per window height change that has
- * classes; the three that read other classes side by side, then the other
- * two), so every word is read and written once per two cells instead of once
+ * classes; the three that read other classes side by side, or as one launch at
+ * low cells, then the other two), so every word is read and written once per two cells instead of once
  * per cell.  Height-capped cells pair up likewise, over the classes within the
- * cap.  32-bit and
- * 64-bit ranks (n >= 23) alike; the static solve (ofp_solve_static) runs the
+ * cap.  32-bit and 64-bit ranks (n >= 23) alike; the static solve (ofp_solve_static) runs the
  * launches one after another.  Results do not depend on it.
  * mode: 0 = off, 1 = on, 2..16 (even) = on with at most that many moduli per
  * launch (default 16).  A context on which it was never called runs pair passes
- * where a launch covers 2^23 words or more (n >= 17) and single cells below.  Walking down a row, cells p and p-1 run
- * as one pair pass when bit p of cell_mask is set (~0u: everywhere), else cell
- * p runs alone; 0 = the library's default (pairs except over cells 4 and 3;
- * the autotuner sets it per size).  Bits 8..9
- * of mode select a kernel variant for 14 or 16 moduli per launch (tuning: bit 8
+ * where a launch covers 2^23 words or more; below 2^25 residues (at most 8
+ * moduli) two cells run as one launch into a second pair of arrays, else
+ * single cells.  Walking down a row, cells p and p-1 run as one pair pass when
+ * bit p of cell_mask is set (~0u: everywhere), else cell p runs alone; 0 = the
+ * library's default (pairs except over cells 3 and 2 and, from 2 to 7 moduli,
+ * 4 and 3; the autotuner sets it per size).  Bits 8..9 of mode select a kernel
+ * variant for 14 or 16 moduli per launch where each window height change has
+ * its own (tuning: bit 8
  * = closure sums gathered before the class's words are loaded, bit 9 = a
  * register budget for three workgroups per CU); results do not depend on it.
  * Other mode bits are refused (group sweeps: ofp_set_group_launch).
