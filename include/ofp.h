@@ -169,9 +169,9 @@ ofp_status ofp_time_cells(ofp_ctx* ctx, float* ms_out, int* kind_out, int capaci
  * library's default (pairs except over cells 3 and 2 and, from 2 to 7 moduli,
  * 4 and 3; the autotuner sets it per size).  Bits 8..9 of mode select a kernel
  * variant for 14 or 16 moduli per launch where each window height change has
- * its own (tuning: bit 8
- * = closure sums gathered before the class's words are loaded, bit 9 = a
- * register budget for three workgroups per CU); results do not depend on it.
+ * its own (tuning: bit 9 = a register budget for three workgroups per CU; bit 8
+ * asks for the closure sums to be gathered before the class's words are loaded,
+ * which these launches do in any case); results do not depend on it.
  * Other mode bits are refused (group sweeps: ofp_set_group_launch).
  * Reference analogue: the reference's fused two-cell group kernels
  * (row6crt20.cu:1033-1154), which run in group scratch. */

@@ -20,8 +20,20 @@ namespace {
 
 using namespace cell;
 
+// Whether the closure sums are gathered before the class's words are loaded (pair_body's
+// GF).  Loading the words first, so that the scans run while they are in flight, keeps up to
+// 14 records per thread live (d = 0: ten words, two sums and, in the scans, four sources):
+// from 14 moduli, or 13 with 64-bit ranks, that is more than the 256 VGPRs two workgroups
+// per CU leave each thread, and up to 65 of them spill.  Gathered first none does.  ms of a
+// full row, words first and sums first: n=20 at 16 moduli 116.5, 113.0; 15 114.1, 112.5; 14
+// 105.6, 105.4; n=21 at 16 310.1, 303.9; 14 277.9, 278.2; with 64-bit ranks n=20 at 16
+// 119.2, 113.4; 14 108.8, 106.1; 13 103.3, 102.1; 12 (two spilled in pair_readers_kernel)
+// 89.2, 89.7.
+template <int KC, typename Idx>
+constexpr int kSumsFirst = KC >= (sizeof(Idx) == 8 ? 13 : 14) ? 1 : 0;
+
 // MB: workgroups of 256 per CU the register allocation must allow (2: at most
-// 256 VGPRs, no spills at 14 moduli; 3: at most 168, with spills).
+// 256 VGPRs, no spills; 3: at most 168, with spills).
 // Capped: the classes of a height-capped pass (a.cap).
 template <int KC, typename Idx, int D, int GF, int MB, bool Capped>
 __global__ __launch_bounds__(256, MB) void pair_kernel(pair::PairLaunch a) {
@@ -77,7 +89,7 @@ __global__ __launch_bounds__(256, 2) void pair_readers_kernel(pair::PairLaunch a
             word[threadIdx.x] = c < a.classes ? pair::decode_class<Idx>(T, ctab, a.W, a.p, c).word : ~0ull;
         }
         for (uint64_t c = lo + threadIdx.x; c < hi; c += blockDim.x)
-            pair::pair_body<KC, Idx, 0, 0>(a, T, decode(0, c), io);
+            pair::pair_body<KC, Idx, 0, kSumsFirst<KC, Idx>>(a, T, decode(0, c), io);
         for (int side = 0; side < 2; ++side) {
             table(2 * side - 1);
             if (threadIdx.x < 2)
@@ -88,8 +100,8 @@ __global__ __launch_bounds__(256, 2) void pair_readers_kernel(pair::PairLaunch a
             __syncthreads();
             const uint64_t b = at[0], e = at[1];
             for (uint64_t c = b + threadIdx.x; c < e; c += blockDim.x) {
-                if (side == 0) pair::pair_body<KC, Idx, -1, 0>(a, T, decode(-1, c), io);
-                else pair::pair_body<KC, Idx, 1, 0>(a, T, decode(1, c), io);
+                if (side == 0) pair::pair_body<KC, Idx, -1, kSumsFirst<KC, Idx>>(a, T, decode(-1, c), io);
+                else pair::pair_body<KC, Idx, 1, kSumsFirst<KC, Idx>>(a, T, decode(1, c), io);
             }
         }
     }
@@ -108,21 +120,15 @@ hipError_t launch_d(const pair::PairLaunch& a, int threads, int blocks, hipStrea
     return hipGetLastError();
 }
 
-// Pair-kernel variant (PairLaunch::variant): bit 0 = gathers first, bit 1 = the
-// three-workgroups-per-CU register budget; only the whole-state 14- and 16-moduli
-// kernels carry the variants (the others run variant 0).
+// Pair-kernel variant (PairLaunch::variant): bit 1 = the three-workgroups-per-CU register
+// budget; only the whole-state 14- and 16-moduli kernels carry it (the others run variant 0).
 template <int KC, typename Idx>
 hipError_t launch_gf(const pair::PairLaunch& a, int threads, int blocks, hipStream_t s) {
-    if (a.cap > 0) return launch_d<KC, Idx, 0, 2, true>(a, threads, blocks, s);
-    if constexpr (KC == 14 || KC == 16) {
-        switch (a.variant & 3) {
-            case 1: return launch_d<KC, Idx, 1, 2>(a, threads, blocks, s);
-            case 2: return launch_d<KC, Idx, 0, 3>(a, threads, blocks, s);
-            case 3: return launch_d<KC, Idx, 1, 3>(a, threads, blocks, s);
-            default: break;
-        }
-    }
-    return launch_d<KC, Idx, 0, 2>(a, threads, blocks, s);
+    constexpr int GF = kSumsFirst<KC, Idx>;
+    if (a.cap > 0) return launch_d<KC, Idx, GF, 2, true>(a, threads, blocks, s);
+    if constexpr (KC == 14 || KC == 16)
+        if (a.variant & 2) return launch_d<KC, Idx, GF, 3>(a, threads, blocks, s);
+    return launch_d<KC, Idx, GF, 2>(a, threads, blocks, s);
 }
 
 // Class tables of every (cap, p, d), cap 0 = none, one wave each (lane = height):

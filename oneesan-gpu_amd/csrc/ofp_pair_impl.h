@@ -145,7 +145,7 @@ struct PairLaunch {
     int cap;           // > 0: only the classes whose P' and S' stay at heights <= cap
     int K, off, kc;    // interleave stride, first modulus, moduli in this launch
     int xcd_shift;
-    int variant;        // kernel variant: bit 0 = gathers first (pair_body's GF), bit 1 = tighter registers
+    int variant;        // kernel variant: bit 1 = tighter registers
     // one launch over every window change d = -3..3 (launch_pair_whole): classes, first
     // workgroup and class table (ct + (d + 3) * ct_bytes) of each
     uint32_t count[7], block[8];
@@ -436,7 +436,8 @@ OFP_HD void closures(const Tab<Idx>& T, int W, int p, const Class<Idx>& k, bool 
 // The pass over one class of window change D.  GF = 0: the class's words are
 // loaded first and the closure scans run while they are in flight; GF = 1: the
 // closure sums (the parts read from memory) are gathered first and the class's
-// words loaded after them, so that fewer values are live during the scans.  Whole:
+// words loaded after them, so that fewer values are live during the scans (kSumsFirst in
+// ofp_pair.hip).  Whole:
 // the pass goes from one pair of arrays to another (io), so the words it keeps are
 // stored too; then no class reads what another writes, in any order.
 template <int KC, typename Idx, int D, int GF = 0, bool Whole = false>
