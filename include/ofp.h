@@ -161,10 +161,10 @@ ofp_status ofp_time_cells(ofp_ctx* ctx, float* ms_out, int* kind_out, int capaci
  * cap.  32-bit and 64-bit ranks (n >= 23) alike; the static solve (ofp_solve_static) runs the
  * launches one after another.  Results do not depend on it.
  * mode: 0 = off, 1 = on, 2..16 (even) = on with at most that many moduli per
- * launch (default 16).  A context on which it was never called runs pair passes
- * where a launch covers 2^23 words or more; below 2^25 residues (at most 8
- * moduli) two cells run as one launch into a second pair of arrays, else
- * single cells.  Walking down a row, cells p and p-1 run as one pair pass when
+ * launch (default 16), -1 = the library's choice, as on a context on which it was
+ * never called: pair passes where a launch covers 2^23 words or more; below 2^25
+ * residues (at most 8 moduli) two cells run as one launch into a second pair of
+ * arrays, else single cells.  Walking down a row, cells p and p-1 run as one pair pass when
  * bit p of cell_mask is set (~0u: everywhere), else cell p runs alone; 0 = the
  * library's default (pairs except over cells 3 and 2 and, from 2 to 7 moduli,
  * 4 and 3; the autotuner sets it per size).  Bits 8..9 of mode select a kernel

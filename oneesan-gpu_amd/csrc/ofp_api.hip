@@ -776,7 +776,7 @@ ofp_status full_rows(ofp_ctx* c, Sweep& s, int rows, int* launches) {
     char key[320];
     snprintf(key, sizeof key, "%p/%p/%d/%d/%d/%d/%d/%d/%d/%d/%d/%d/%d/%d/%u", (void*)s.main, (void*)s.blk, s.n, s.K,
              c->threads, c->blocks_per_cu, s.layout, c->low_cells, c->low_kc, c->variant * 100 + c->sorted_from,
-             c->xcd_shift, c->index_bits, pairs ? 1 + c->pair_variant : 0, c->pair_kc, c->pair_mask);
+             c->xcd_shift, c->index_bits, pairs ? 1 + c->pair_variant + 4 * (c->pair_rows + 1) : 0, c->pair_kc, c->pair_mask);
     std::string k = key;
     for (uint32_t m : s.mods) k += "/" + std::to_string(m);
     if (k != s.row_key || !s.row_exec) {
@@ -1434,15 +1434,18 @@ ofp_status ofp_time_cells(ofp_ctx* c, float* ms_out, int* kind_out, int capacity
 
 ofp_status ofp_set_pair_passes(ofp_ctx* c, int mode, uint32_t cell_mask) {
     if (!c) return OFP_E_ARG;
+    const bool library = mode == -1;  // as on a fresh context
+    if (library) mode = 1;
     // mode bits 8..9 select the pair-kernel variant (tuning)
     if (mode & ~0x3ff) return fail(c, OFP_E_ARG, "pair passes: unknown mode bits (group sweeps: ofp_set_group_launch)");
     const int variant = (mode >> 8) & 3;
     mode &= 0xff;
     if (mode < 0 || mode > kMaxKC || (mode > 1 && (mode & 1)))
-        return fail(c, OFP_E_ARG, "pair passes: 0 (off), 1 (on) or an even moduli count per launch up to 16");
+        return fail(c, OFP_E_ARG, "pair passes: -1 (the library's choice), 0 (off), 1 (on) or an even moduli count "
+                                  "per launch up to 16");
     if (variant != c->pair_variant) drop_graph(c->st);
     c->pair_variant = variant;
-    const int on = mode > 0 ? 1 : 0;  // asked for: at every size
+    const int on = library ? -1 : mode > 0 ? 1 : 0;  // asked for: at every size
     if (on != c->pair_rows) drop_graph(c->st);
     c->pair_rows = on;
     c->pair_kc = mode > 1 ? mode : kMaxKC;

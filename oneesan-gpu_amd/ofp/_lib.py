@@ -409,9 +409,9 @@ class Context:
 
     def set_pair_passes(self, mode: bool | int, cell_mask: int = 0) -> None:
         """Whole-state rows as pair passes (two cells per in-place pass) instead of
-        one launch per cell: False/0 off, True/1 on (a fresh context: on from 2^23 words
-        per launch), an even 2..16 = on with at most
-        that many moduli per launch; cells p and p-1 pair up where bit p of
+        one launch per cell: False/0 off, True/1 on, an even 2..16 = on with at most
+        that many moduli per launch, -1 = the library's choice by size, as on a fresh
+        context; cells p and p-1 pair up where bit p of
         cell_mask is set (0: the library's default).  Bits 8..9 of an int mode pick
         a kernel variant."""
         m = int(mode) if not isinstance(mode, bool) else (1 if mode else 0)

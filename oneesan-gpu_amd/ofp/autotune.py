@@ -5,8 +5,10 @@ For a given (n, k) it prepares the device state once, then times row sweeps
 and keeps the fastest.  Timing runs advance the state, which does not change
 the cost of a row as long as height caps are off (they are, for these stages).
 A last stage picks the height-cap threshold on the first rows of a solve, the
-ones caps shorten.  Results persist in a JSON cache keyed by device name, n
-and k, so a solver or the serving loop can look them up without re-tuning.
+ones caps shorten.  Then whole solves are timed with the settings found and with the
+library's own choices, which those of a row only replace where they are faster
+(choose_stage).  Results persist in a JSON cache keyed by n and k, so a solver or
+the serving loop can look them up without re-tuning.
 
 Reference analogue: scripts/run/autotune.py:28 (the reference tunes its
 frontier thread count and batch limits by re-running the solver binary);
@@ -40,6 +42,11 @@ SORTED_FROM = (0, 4, 6, 8, 12)
 # timed on rows 1..CAPPED_ROWS of a solve (every row the forward bound caps at n <= 22)
 CAP_PERCENTS = (75, 85, 95)
 CAPPED_ROWS = 12
+# the library's own launch settings (the height caps' depend on the moduli count)
+DEFAULTS = {"layout": 1, "threads": 256, "blocks_per_cu": 32, "variant": 2, "low_cells": 0, "low_kc": 16,
+            "xcd_shift": 5, "sorted_from": -1}
+# a setting replaces the library's where whole solves are faster by more than runs differ
+CHOICE_GAIN = 0.02
 
 
 def _key(n: int, k: int) -> str:
@@ -79,7 +86,7 @@ def lookup(n: int, k: int, path: Path = DEFAULT_CACHE) -> dict | None:
 
 
 def pair_mask_for(n: int, k: int, path: Path = DEFAULT_CACHE) -> int:
-    """The pair mask to run (n, k) with: the one tuned for (n, k), else for the
+    """The pair mask the tables hold for (n, k): the one tuned for (n, k), else for the
     same n and the nearest moduli count (one modulus or several first), else 0
     (the library's default).  A mask names cell positions, which shift with n, so
     one tuned at another n does not carry over."""
@@ -97,19 +104,73 @@ def pair_mask_for(n: int, k: int, path: Path = DEFAULT_CACHE) -> int:
     return 0
 
 
+def pair_settings(n: int, k: int, path: Path = DEFAULT_CACHE) -> tuple[int, int]:
+    """(mode, cell mask) of the pair passes to run (n, k) with: the table's where its
+    entry of this very (n, k) was timed against the library's choice on whole solves
+    and was faster, else the library's choice (-1, 0).  Which form two cells take
+    depends on n and k, so another size's entry says nothing here."""
+    for table in (load_cache(path), load_cache(PACKAGED)):
+        ent = table.get(_key(n, k))
+        if ent:
+            if ent.get("pair_choice") == "table":
+                return int(ent.get("pair_mode", 1)), pair_mask_for(n, k, path)
+            break
+    return -1, 0
+
+
+def _set(ctx: "_lib.Context", ent: dict, pairs: tuple[int, int]) -> None:
+    ctx.set_layout(int(ent.get("layout", 1)))
+    ctx.set_launch(int(ent["threads"]), int(ent["blocks_per_cu"]))
+    ctx.set_variant(int(ent.get("variant", 2)))
+    ctx.set_low_cells(int(ent.get("low_cells", 0)), int(ent.get("low_kc", 16)))
+    ctx.set_height_caps(int(ent.get("cap_percent", _lib.DEFAULT_CAP_PERCENT)))
+    ctx.set_xcd_pieces(int(ent.get("xcd_shift", 5)))
+    ctx.set_sorted_cells(int(ent.get("sorted_from", -1)))
+    ctx.set_pair_passes(*pairs)
+
+
 def apply(ctx: "_lib.Context", n: int, k: int) -> dict | None:
     """Set the best known launch shape and layout on ctx (before prepare/solve)."""
     ent = lookup(n, k)
     if ent:
-        ctx.set_layout(int(ent.get("layout", 1)))
-        ctx.set_launch(int(ent["threads"]), int(ent["blocks_per_cu"]))
-        ctx.set_variant(int(ent.get("variant", 2)))
-        ctx.set_low_cells(int(ent.get("low_cells", 0)), int(ent.get("low_kc", 16)))
-        ctx.set_height_caps(int(ent.get("cap_percent", _lib.DEFAULT_CAP_PERCENT)))
-        ctx.set_xcd_pieces(int(ent.get("xcd_shift", 5)))
-        ctx.set_sorted_cells(int(ent.get("sorted_from", -1)))
-        ctx.set_pair_passes(int(ent.get("pair_mode", 1)), pair_mask_for(n, k))
+        _set(ctx, ent, pair_settings(n, k))
     return ent
+
+
+def solve_ms(ctx: "_lib.Context", n: int, moduli: list[int]) -> float:
+    """Time of one whole solve: the least of up to seven after a first one."""
+    ctx.solve(n, moduli)
+    best, spent = float("inf"), 0.0
+    for _ in range(7):
+        t0 = time.perf_counter()
+        ctx.solve(n, moduli)
+        el = time.perf_counter() - t0
+        best, spent = min(best, el), spent + el
+        if spent > 3.0:
+            break
+    return best * 1e3
+
+
+def choose_stage(ctx: "_lib.Context", n: int, moduli: list[int], ent: dict, log=None) -> dict:
+    """What whole solves of (n, moduli) should run with: the library's own settings; ent's
+    launch settings with the library's pair choice; those with ent's pair settings.
+    The earlier one stands unless a later one is faster by CHOICE_GAIN.  Returns ent
+    with the launch settings chosen, `pair_choice` and `solve_ms`; sets them on ctx."""
+    k = len(moduli)
+    own = dict(ent, **DEFAULTS, cap_percent=75 if k == 1 else 85)
+    tuned = (int(ent.get("pair_mode", 1)), int(ent.get("pair_mask", 0)))
+    cands = [(own, (-1, 0), "library"), (ent, (-1, 0), "library"), (ent, tuned, "table")]
+    best = None
+    for e, pairs, choice in cands:
+        _set(ctx, e, pairs)
+        ms = solve_ms(ctx, n, moduli)
+        if log:
+            log(f"autotune n={n} k={k} {'library' if e is own else 'tuned'} launches, {choice} pairs: {ms:.3f} ms")
+        if best is None or ms < best[0] * (1.0 - CHOICE_GAIN):
+            best = (ms, e, pairs, choice)
+    ms, e, pairs, choice = best
+    _set(ctx, e, pairs)
+    return dict(e, pair_choice=choice, solve_ms=ms)
 
 
 def pair_stage(ctx: "_lib.Context", n: int, moduli: list[int], log=None) -> tuple[int, float]:
@@ -145,7 +206,8 @@ def pair_stage(ctx: "_lib.Context", n: int, moduli: list[int], log=None) -> tupl
 def tune(ctx: "_lib.Context", n: int, moduli: list[int], rows: int = 1,
          threads: Iterable[int] = THREADS, blocks_per_cu: Iterable[int] = BLOCKS_PER_CU,
          layouts: Iterable[int] = LAYOUTS, path: Path | None = DEFAULT_CACHE, log=None) -> dict:
-    """Time every (layout, launch shape); set the best on ctx; return the table."""
+    """Time every (layout, launch shape), then whole solves with the best and with the
+    library's own settings; set what is fastest on ctx; return the table."""
     table = []
     best = None
     ctx.set_height_caps(0)
@@ -179,7 +241,7 @@ def tune(ctx: "_lib.Context", n: int, moduli: list[int], rows: int = 1,
     if best["layout"] == 1:
         ctx.prepare(n, moduli)
         for var in VARIANTS:
-            for lc, lk in (LOW_CELLS if len(moduli) > 1 else ((0, 16),)):
+            for lc, lk in ((lc, lk) for lc, lk in LOW_CELLS if lc == 0 or lk < len(moduli)):
                 ctx.set_variant(var)
                 ctx.set_low_cells(lc, lk)
                 ctx.row_sweep(1)
@@ -250,7 +312,7 @@ def tune(ctx: "_lib.Context", n: int, moduli: list[int], rows: int = 1,
                 log(f"autotune n={n} k={len(moduli)} cap_percent={pct}: rows 1..{rows_capped} "
                     f"{timed[pct]:.2f} ms/row")
         best["cap_percent"] = min(timed, key=timed.get)
-    ctx.set_height_caps(best["cap_percent"])
+    best = choose_stage(ctx, n, moduli, best, log)
     result = {"best": best, "table": table}
     if path is not None:
         data = load_cache(path)
@@ -262,6 +324,7 @@ def tune(ctx: "_lib.Context", n: int, moduli: list[int], rows: int = 1,
                                       "xcd_shift": best["xcd_shift"],
                                       "sorted_from": best["sorted_from"],
                                       "pair_mode": best["pair_mode"], "pair_mask": best["pair_mask"],
+                                      "pair_choice": best["pair_choice"], "solve_ms": best["solve_ms"],
                                       "row_ms": best["row_ms"], "tuned_at": time.time()}
         save_cache(data, path)
     return result

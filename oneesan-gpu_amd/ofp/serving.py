@@ -171,6 +171,8 @@ class Server:
                 nxt = reqs[i].arrival - now() if i < len(reqs) else poll_s
                 time.sleep(max(0.0, min(poll_s, nxt)))
         wall = now()
+        if self.tuned:  # the last job's pair settings are not the next solve's
+            self.ctx.set_pair_passes(-1)
         lat = sorted(r.latency for r in reqs)
         residues = sum(len(r.moduli) for r in reqs)
 
