@@ -83,8 +83,7 @@ struct Sum {
     }
     // The workgroup's sums (of moduli off..) into one of the kCopies sets of
     // accumulators: per modulus the low sums, and the high sums in two halves (a
-    // workgroup's stay below 2^63: a lane adds at most 2^13 products of a residue and
-    // a sum below 2^43), reduced by the last kernel.
+    // workgroup's cannot wrap: block_sum), reduced by the last kernel.
     template <int NT>
     __device__ void flush(const GlueLaunch& a, int off) {
         __shared__ unsigned long long part[NT / 64][2 * KC];
@@ -350,7 +349,7 @@ __global__ __launch_bounds__(256) void glue_big_kernel(GlueLaunch a) {
 }
 
 // The answer word (index 0) takes the sums, one wave per modulus: low + 2^32 (mid +
-// 2^32 high), each below 2^63 over all waves.
+// 2^32 high), each below 2^64 over all waves.
 __global__ __launch_bounds__(64) void glue_finish_kernel(GlueLaunch a, uint32_t* main) {
     const int j = (int)blockIdx.x, lane = (int)threadIdx.x;
     const uint64_t m = a.mods ? a.mods[j] : a.mod[j];
@@ -547,21 +546,21 @@ hipError_t launch_lds(const GlueLaunch& a, uint32_t blocks, hipStream_t s) {
                                                  (int)bytes);
         if (e != hipSuccess) return e;
     }
-    const uint32_t passes = (uint32_t)(a.K + KC - 1) / KC;  // blocks: whole rounds of 8 XCDs and all passes
-    hipLaunchKernelGGL(k, dim3(std::max(1u, blocks / (8 * passes)) * 8 * passes), dim3(NT), bytes, s, a);
+    hipLaunchKernelGGL(k, dim3(blocks), dim3(NT), bytes, s, a);
     return hipGetLastError();
 }
 
 template <typename Idx, int NT, int TW>
-hipError_t launch_lds_kc(GlueLaunch a, int most, uint32_t blocks, hipStream_t s) {
-    const int kc = std::min(most, a.K >= 4 ? 4 : (a.K >= 2 ? 2 : 1));
+hipError_t launch_lds_kc(GlueLaunch a, const Shape& sh, hipStream_t s) {
     uint32_t rows = 0;
     for (int i = 0; i < a.segs; ++i) rows = std::max(rows, a.seg[i].rows);
-    a.ystride = round_up((rows + 1) * kc * 4, 16);
-    switch (kc) {
-        case 1: return launch_lds<1, Idx, NT, TW>(a, blocks, s);
-        case 2: return launch_lds<2, Idx, NT, TW>(a, blocks, s);
-        default: return launch_lds<4, Idx, NT, TW>(a, blocks, s);
+    a.tasks = sh.tasks;
+    a.piece = sh.piece;
+    a.ystride = round_up((rows + 1) * sh.kc * 4, 16);
+    switch (sh.kc) {
+        case 1: return launch_lds<1, Idx, NT, TW>(a, sh.blocks, s);
+        case 2: return launch_lds<2, Idx, NT, TW>(a, sh.blocks, s);
+        default: return launch_lds<4, Idx, NT, TW>(a, sh.blocks, s);
     }
 }
 
@@ -605,11 +604,6 @@ hipError_t launch_idx(GlueLaunch a, const Tables* tabs, const Ballot& hb, const 
         g.count = binom[a.W * 32 + m];
         return g;
     };
-    // the strand counts of one launch, the most strands (the longest tasks) first
-    struct Class {
-        int lo, hi;
-    };
-    static const Class kClasses[] = {{19, 19}, {17, 17}, {13, 15}, {1, 11}};
     const int top = a.W % 2 ? a.W : a.W - 1;
     hipError_t e = hipSuccess;
     for (int m = top; m > kTabStrands && e == hipSuccess; m -= 2) {
@@ -631,22 +625,12 @@ hipError_t launch_idx(GlueLaunch a, const Tables* tabs, const Ballot& hb, const 
     for (const Class& c : kClasses) {
         if (e != hipSuccess) break;
         a.segs = 0;
-        a.tasks = 0;
-        for (int m = std::min(c.hi, top); m >= c.lo; m -= 2) {
-            a.seg[a.segs] = seg_of(m);
-            a.tasks += a.seg[a.segs++].count;
-        }
-        if (!a.tasks) continue;
-        a.piece = std::min(32u, std::max(1u, a.tasks / (64u * (c.hi <= 11 ? 4u : 1u))));
-        // resident workgroups (the LDS and registers of a class), fewer where a team
-        // would get less than two tasks per pass
-        const uint32_t cu = (uint32_t)cus;
-        const auto blocks = [&](uint32_t most, uint32_t teams) {
-            return std::min(most, std::max(cu, (a.tasks + 2 * teams - 1) / (2 * teams) * (uint32_t)((a.K + 3) / 4)));
-        };
-        if (c.lo >= 17) e = launch_lds_kc<Idx, 1024, 16>(a, c.lo == 19 ? 2 : 4, blocks(cu * 2, 1), s);
-        else if (c.lo >= 13) e = launch_lds_kc<Idx, 256, 4>(a, 4, blocks(cu * 8, 1), s);
-        else e = launch_lds_kc<Idx, 256, 1>(a, 4, blocks(cu * 8, 4), s);
+        for (int m = std::min(c.hi, top); m >= c.lo; m -= 2) a.seg[a.segs++] = seg_of(m);
+        const Shape sh = class_shape(c, a.W, a.K, cus, binom);
+        if (!sh.tasks) continue;
+        if (c.lo >= 17) e = launch_lds_kc<Idx, 1024, 16>(a, sh, s);
+        else if (c.lo >= 13) e = launch_lds_kc<Idx, 256, 4>(a, sh, s);
+        else e = launch_lds_kc<Idx, 256, 1>(a, sh, s);
         if (launches) ++*launches;
     }
     return e;

@@ -43,6 +43,8 @@
 // odd row with position c empty, where u[w] + 2 ublocked[w] takes the place of
 // u[w] on one side and both orders are summed.
 #pragma once
+#include <algorithm>
+
 #include "ofp_cell_impl.h"
 
 namespace ofp {
@@ -193,6 +195,63 @@ constexpr uint32_t kLongest[] = {1, 1, 2, 4, 10, 24, 66, 174, 504, 1406};
 inline uint32_t chunk_bound(int m, uint32_t rows) {
     const uint32_t i = (uint32_t)(m - 1) / 2;
     return kOnes[i] / 512 + kLongest[i] / 8 + (rows + 63) / 64 + 2;
+}
+
+// ---- launches of the tasks in LDS (glue_kernel) ----
+// The strand counts of one launch, the most strands (the longest tasks) first: waves of a
+// workgroup, waves sharing a task, most moduli per pass, resident workgroups per CU.
+struct Class {
+    int lo, hi, waves, team;
+    int most_kc;
+    uint32_t per_cu;
+};
+constexpr Class kClasses[] = {{19, 19, 16, 16, 2, 2}, {17, 17, 16, 16, 4, 2}, {13, 15, 4, 4, 4, 8}, {1, 11, 4, 1, 4, 8}};
+constexpr double kSumLimit = 18446744073709551616.0;  // 2^64: the sums are unsigned
+
+// One launch: teams of a workgroup, moduli of a pass, tasks, tasks of a piece per team
+// (pieces go to the 8 XCDs in turn), passes and blocks (per pass and XCD: blocks / 8 / passes).
+struct Shape {
+    uint32_t teams, kc, tasks, piece, passes, blocks;
+};
+
+// No more than this many of `count` consecutive tasks go to one XCD ...
+inline uint64_t xcd_tasks(const Shape& s, uint64_t count) {
+    const uint64_t P = (uint64_t)s.piece * s.teams;
+    return std::min<uint64_t>(count, ((count + 8 * P - 1) / (8 * P) + 1) * P);
+}
+// ... and this many of them to one of its blocks of a pass, which takes a round of `teams`
+// neighbouring ones in every (blocks / 8 / passes).
+inline uint64_t block_tasks(const Shape& s, uint64_t count) {
+    const uint64_t round = (uint64_t)(s.blocks / 8 / s.passes) * s.teams;
+    return std::min<uint64_t>(xcd_tasks(s, count), ((xcd_tasks(s, count) + round - 1) / round + 1) * s.teams);
+}
+// Greatest sum of the high halves of a block's products: a task of m strands adds
+// kOnes[m / 2] products of two residues, whose high halves are below 2^32 each.  (The low
+// halves are fewer, one per word.)
+inline double block_sum(const Shape& s, const Class& c, int W, const uint32_t* bin) {
+    double sum = 0;
+    for (int m = c.lo; m <= c.hi && m <= W; m += 2)
+        sum += (double)block_tasks(s, bin[W * 32 + m]) * kOnes[(m - 1) / 2] * 4294967296.0;
+    return sum;
+}
+
+// The launch of class c at width W with records of K moduli on cus CUs: the resident
+// workgroups (the LDS and registers of a class), fewer where a team would get less than
+// two tasks per pass, more where a block's 64-bit sums could wrap (few CUs, or many passes:
+// with 256 CUs at W = 24 from 11 moduli on).
+inline Shape class_shape(const Class& c, int W, int K, int cus, const uint32_t* bin) {
+    Shape s{};
+    s.teams = (uint32_t)(c.waves / c.team);
+    s.kc = (uint32_t)std::min(c.most_kc, K >= 4 ? 4 : (K >= 2 ? 2 : 1));
+    for (int m = c.lo; m <= c.hi && m <= W; m += 2) s.tasks += bin[W * 32 + m];
+    s.piece = std::min(32u, std::max(1u, s.tasks / (64u * s.teams)));
+    s.passes = ((uint32_t)K + s.kc - 1) / s.kc;
+    const uint32_t few = (s.tasks + 2 * s.teams - 1) / (2 * s.teams) * (((uint32_t)K + 3) / 4);
+    const uint32_t blocks = std::min((uint32_t)cus * c.per_cu, std::max((uint32_t)cus, few));
+    // whole rounds of 8 XCDs and all passes
+    s.blocks = std::max(1u, blocks / (8 * s.passes)) * 8 * s.passes;
+    while (block_sum(s, c, W, bin) >= kSumLimit) s.blocks *= 2;
+    return s;
 }
 
 }  // namespace glue
