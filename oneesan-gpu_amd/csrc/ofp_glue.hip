@@ -221,10 +221,7 @@ __global__ __launch_bounds__(NT) void glue_kernel(GlueLaunch a) {
 }
 
 // ---- strands beyond the lists ----
-// Scratch of a task (a.each entries of K residues): the lower words (rows of m
-// strands), then one array of m - 2 strands per place b = 0..m-2 of the arc removed
-// first, then, for m = kTabStrands + 4, one of m - 4 strands per pair (b, b2), b2 <
-// b: the arc removed next lies below the first one's place or around it.
+// Entry i of a task's scratch (a.each of K residues; laid out as pull_entry says).
 __device__ __forceinline__ uint32_t* entry(const GlueLaunch& a, uint32_t task, uint32_t i) {
     return a.scratch + ((uint64_t)task * a.each + i) * (uint32_t)a.K;
 }
@@ -258,33 +255,23 @@ __global__ __launch_bounds__(256) void glue_pull_kernel(GlueLaunch a, uint32_t a
     __shared__ Ballot b;
     load_ballot(b, a.ballot);
     __syncthreads();
-    const int M = a.seg[0].m - 2 * a.removed;
-    const uint32_t rows = b.n[M - 2][1];
+    const int m = a.seg[0].m;
+    const uint32_t rows = b.n[m - 2 * a.removed - 2][1];
     const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
     const uint32_t ta = (uint32_t)(i / rows), l = (uint32_t)(i - (uint64_t)ta * rows);
     const uint32_t t = ta / arrays, node = ta - t * arrays;
     if (t >= a.batch) return;
-    if (!mask_weight(mask_of(a.binom, a.W, a.seg[0].m, a.task0 + t), a.W, a.center)) return;
-    // the array's place(s): first level b = node; second level the pairs b2 < b in
-    // the order b (b - 1) / 2 + b2
-    int place = (int)node;
-    uint32_t src = a.from;
-    if (a.removed) {
-        int b1 = 1;
-        while ((uint32_t)(b1 * (b1 + 1) / 2) <= node) ++b1;
-        place = (int)node - b1 * (b1 - 1) / 2;
-        src += (uint32_t)b1 * b.n[M][1];
-        if (place > M - 2) return;  // no such place: never read
-    }
+    if (!mask_weight(mask_of(a.binom, a.W, m, a.task0 + t), a.W, a.center)) return;
     const int off = (int)blockIdx.y * KC;
     uint32_t mod[KC], sum[KC] = {};
     load_mods<KC>(a, off, mod);
-    preimages(M, labels_of(b, M - 2, l), M - 2 - place, [&](uint32_t lab) {
+    const bool place = pull_entry(b, m, a.removed, a.from, node, l, [&](uint32_t src) {
         uint32_t e[KC];
-        load_rec<KC>(entry(a, t, src), rank_of(b, M, lab), a.K, off, e);
+        load_rec<KC>(entry(a, t, src), 0, a.K, off, e);
 #pragma unroll
         for (int j = 0; j < KC; ++j) sum[j] = addm(sum[j], e[j], mod[j]);
     });
+    if (!place) return;
     uint32_t* out = entry(a, t, a.to + node * rows + l) + off;
 #pragma unroll
     for (int j = 0; j < KC; ++j)
@@ -318,14 +305,7 @@ __global__ __launch_bounds__(256) void glue_big_kernel(GlueLaunch a) {
         uint32_t lab = labels_of(b, g.m, l);
         uint32_t x[KC];
         load_upper<KC, Idx>(a, D, occ, lab, weight, off, mod, x);
-        const int b1 = top_arc(lab);
-        lab = without_pair(lab, b1);
-        uint32_t node = (uint32_t)b1;
-        if (g.m > kTabStrands + 2) {
-            const int b2 = top_arc(lab);
-            lab = without_pair(lab, b2);
-            node = (uint32_t)(b1 * (b1 - 1) / 2 + b2);
-        }
+        const uint32_t node = upper_node(g.m, kTabStrands, lab);
         const uint32_t* y = entry(a, t, a.from + node * lists.rows);
         const uint32_t slot = lists.slot[rank_of(b, kTabStrands, lab)], s = slot >> 6;
         const uint4* cols = lists.cols + (slot & 63u);
@@ -564,13 +544,6 @@ hipError_t launch_lds_kc(GlueLaunch a, const Shape& sh, hipStream_t s) {
     }
 }
 
-// Scratch entries of one task of m strands.
-uint32_t task_entries(const Ballot& b, int m) {
-    uint32_t n = b.n[m][1] + (uint32_t)(m - 1) * b.n[m - 2][1];
-    if (m > kTabStrands + 2) n += (uint32_t)((m - 1) * (m - 2) / 2) * b.n[m - 4][1];
-    return n;
-}
-
 template <int KC, typename Idx>
 hipError_t launch_big_kc(GlueLaunch a, const Ballot& hb, hipStream_t s, int* launches) {
     const int m = a.seg[0].m;
@@ -581,7 +554,7 @@ hipError_t launch_big_kc(GlueLaunch a, const Ballot& hb, hipStream_t s, int* lau
     a.to = hb.n[m][1];
     const int levels = (m - kTabStrands) / 2;  // 1 or 2
     for (int r = 0; r < levels; ++r) {
-        const uint32_t arrays = r == 0 ? (uint32_t)(m - 1) : (uint32_t)((m - 1) * (m - 2) / 2), rows = hb.n[m - 2 * r - 2][1];
+        const uint32_t arrays = level_arrays(m, r), rows = hb.n[m - 2 * r - 2][1];
         a.removed = r;
         hipLaunchKernelGGL((glue_pull_kernel<KC>), dim3(grid((uint64_t)a.batch * arrays * rows), passes), dim3(256), 0, s, a,
                            arrays);
@@ -610,7 +583,7 @@ hipError_t launch_idx(GlueLaunch a, const Tables* tabs, const Ballot& hb, const 
         a.segs = 1;
         a.seg[0] = seg_of(m);
         a.seg[1] = seg_of(kTabStrands);
-        a.each = task_entries(hb, m);
+        a.each = task_entries(hb, m, kTabStrands);
         const Seg& g = a.seg[0];
         const uint32_t most =
             (uint32_t)std::min<uint64_t>(256, std::max<uint64_t>(1, scratch_bytes / ((uint64_t)a.each * a.K * 4)));
@@ -641,7 +614,7 @@ hipError_t launch_idx(GlueLaunch a, const Tables* tabs, const Ballot& hb, const 
 size_t scratch_need(const Ballot& hb, int W, int K) {
     const int top = W % 2 ? W : W - 1;
     if (top <= kTabStrands) return 0;
-    return std::max<size_t>((size_t)64 << 20, (size_t)task_entries(hb, top) * K * 4);
+    return std::max<size_t>((size_t)64 << 20, (size_t)task_entries(hb, top, kTabStrands) * K * 4);
 }
 
 hipError_t launch_glue(const GlueLaunch& a, const Tables* tabs, const Ballot& hb, const uint32_t* binom, bool wide, int cus,

@@ -186,6 +186,46 @@ OFP_HD uint32_t preimage_count(int m, uint32_t v, int j) {
     return n;
 }
 
+// ---- strands beyond the lists: the scratch of a task ----
+// Entries of a task of m strands whose words are listed at `tab` strands (m = tab + 2 or
+// tab + 4): the lower words (n[m][1]), then one array of m - 2 strands per place b =
+// 0..m-2 of the arc removed first, then, for m = tab + 4, one of m - 4 strands per pair
+// (b, b2), b2 < b: the arc removed next lies below the first one's place or around it.
+OFP_HD uint32_t pair_node(int b, int b2) { return (uint32_t)(b * (b - 1) / 2 + b2); }
+OFP_HD uint32_t level_arrays(int m, int removed) { return removed == 0 ? (uint32_t)(m - 1) : pair_node(m - 1, 0); }
+inline uint32_t task_entries(const Ballot& b, int m, int tab) {
+    uint32_t n = b.n[m][1];
+    for (int r = 0; r < (m - tab) / 2; ++r) n += level_arrays(m, r) * b.n[m - 2 * r - 2][1];
+    return n;
+}
+// Entry l of array `node` one level down, `removed` (0 or 1) arcs being gone from the m
+// strands of the level read, which begins at entry `from`: add(index) for each preimage
+// there.  False: no such place, the entry is never read.
+template <class Add>
+OFP_HD bool pull_entry(const Ballot& b, int m, int removed, uint32_t from, uint32_t node, uint32_t l, Add&& add) {
+    const int M = m - 2 * removed;  // strands of the level read
+    int place = (int)node;
+    if (removed) {
+        int b1 = 1;
+        while (pair_node(b1 + 1, 0) <= node) ++b1;
+        place = (int)(node - pair_node(b1, 0));
+        if (place > M - 2) return false;
+        from += (uint32_t)b1 * b.n[M][1];
+    }
+    preimages(M, labels_of(b, M - 2, l), M - 2 - place, [&](uint32_t lab) { add(from + rank_of(b, M, lab)); });
+    return true;
+}
+// The array (at the last level) in which an upper word's list is summed; lab becomes the
+// labels left at `tab` strands.
+OFP_HD uint32_t upper_node(int m, int tab, uint32_t& lab) {
+    const int b1 = top_arc(lab);
+    lab = without_pair(lab, b1);
+    if (m <= tab + 2) return (uint32_t)b1;
+    const int b2 = top_arc(lab);
+    lab = without_pair(lab, b2);
+    return pair_node(b1, b2);
+}
+
 // Ones of G_m (open meanders with m crossings) and the most in a row, m = 1, 3, ...
 constexpr uint32_t kOnes[] = {1, 2, 8, 42, 262, 1828, 13820, 110954, 933458, 8152860};
 constexpr uint32_t kLongest[] = {1, 1, 2, 4, 10, 24, 66, 174, 504, 1406};
