@@ -56,7 +56,7 @@ typedef struct ofp_plan_info {
     uint64_t blocked_states;  /* H_DP[W-1][1] */
     uint64_t state_bytes;     /* device bytes of the interleaved state for k moduli */
     uint64_t transitions;     /* W*(W-1)*(main+blocked)*k: frontier transitions per solve */
-    uint64_t free_bytes;      /* free HBM on the device right now */
+    uint64_t free_bytes;      /* free HBM on the device right now, and what the context would give up */
     int fits;                 /* state_bytes + reserve <= free_bytes */
 } ofp_plan_info;
 
@@ -109,6 +109,15 @@ ofp_status ofp_solve_static(ofp_ctx* ctx, int n, const uint32_t* moduli, int k,
  * as fit.  Reference analogue: its residue loop runs one modulus per sweep
  * (row6crt20.cu:1784-1841). */
 ofp_status ofp_set_max_batch(ofp_ctx* ctx, int max_moduli);
+
+/* What solves and jobs may hold beside their state: 1 (default) = what makes them
+ * faster where it fits (a second pair of arrays for small states, the scratch of a
+ * half-row solve's last step from n = 20 up), 0 = the state and a few KB only.  Read
+ * when a state is set up and when its rows are enqueued.  Residues do not depend on it. */
+ofp_status ofp_set_extra_memory(ofp_ctx* ctx, int on);
+/* The most that a solve or job of (n, k) in the state-major layout holds beside
+ * ofp_plan's state_bytes.  Host-only, no GPU; 0 for arguments out of range. */
+uint64_t ofp_extra_bytes(int n, int k);
 
 /* The sweeps ofp_solve makes of k moduli with at most max_per_sweep each:
  * fewest sweeps, near-equal sizes, even sizes where that adds no sweep.
@@ -268,7 +277,7 @@ typedef struct ofp_job ofp_job;
 typedef struct ofp_job_info {
     int n, k, rows_total, rows_enqueued;
     int idle;                      /* 1 when all enqueued work has finished */
-    uint64_t state_bytes;          /* device bytes held by the job */
+    uint64_t state_bytes;          /* device bytes held by the job (its state and what it holds beside it) */
     uint64_t transitions_per_row;
 } ofp_job_info;
 /* Allocate and initialise the state; fails with OFP_E_MEMORY if it does not fit. */

@@ -98,6 +98,7 @@ struct ofp_ctx {
                            // -1: from cell 6 for launches of 8 or more moduli, else none)
     int index_bits = 0;    // 0: 32-bit ranks for W <= 23, 64-bit above; 64: 64-bit ranks always
     int max_batch = 0;     // moduli per sweep of ofp_solve (0: as many as fit HBM)
+    bool extra_memory = true;  // solves may hold more than their state (ofp_set_extra_memory)
     char* win = nullptr;   // window buffer of shard and group sweeps, reused from call to call
     size_t win_bytes = 0;
     // The LOW window the last group sweep left in `win` (what ofp_group_exchange reads).
@@ -273,6 +274,21 @@ int grid_blocks(const ofp_ctx* c, uint64_t nblk) {
     return (int)std::max<uint64_t>(b, 8);
 }
 
+// What the context holds beside its own state and could do without, given up where
+// another buffer does not fit otherwise: the copy buffer, the scratch of the last solve's
+// last step and a small state's second pair of arrays (its rows run as above that size).
+uint64_t spare_bytes(const ofp_ctx* c) { return c->io_bytes + c->st.main2_cap + c->st.blk2_cap + c->st.gscratch_cap; }
+void release_spare(ofp_ctx* c) {
+    if (c->io) (void)hipFree(c->io);
+    c->io = nullptr;
+    c->io_bytes = 0;
+    free_second(c->st);
+    c->st.whole = false;
+    sweep_free(c->st, c->st.gscratch);
+    c->st.gscratch = nullptr;
+    c->st.gscratch_cap = 0;
+}
+
 // The window buffer of shard and group sweeps: kept from call to call, so that
 // streaming windows of one size through HBM neither frees a touched buffer nor
 // touches fresh pages per window (each costs about a second per 100 GB).
@@ -296,6 +312,10 @@ ofp_status window_buffer(ofp_ctx* c, size_t bytes, char** out) {
         OFP_HIP(c, hipFree(c->stage), "free exchange buffer");
         c->stage = nullptr;
         c->stage_bytes = 0;
+        OFP_HIP(c, hipMemGetInfo(&fr, &tot), "hipMemGetInfo");
+    }
+    if (bytes + c->reserve > fr && spare_bytes(c)) {
+        release_spare(c);
         OFP_HIP(c, hipMemGetInfo(&fr, &tot), "hipMemGetInfo");
     }
     if (bytes + c->reserve > fr) return fail(c, OFP_E_MEMORY, "window does not fit HBM");
@@ -330,7 +350,6 @@ struct Carve {
     }
 };
 
-// Ensure device buffers of s for (n, moduli) in the context's current layout.
 // Whether n in the context's settings runs its full rows as pair passes: pair
 // mode on, state-major layout, at least two cells (32-bit ranks for n <= 22,
 // 64-bit above or when forced).
@@ -352,15 +371,39 @@ constexpr uint64_t kPairWords = 1ull << 23;
 // 8.95, 10.0; n=18 at one (4.4e7) 14.5, 15.8.  More than kWholeKC moduli would take two
 // launches a pass, each with the index math of one: n=15 at 12 3.70, 5.01.
 constexpr uint64_t kWholeWords = 1ull << 25;
+constexpr int kHalfMinW = 4;  // solves of fewer columns run all their rows (half_ready)
 
-// Whether n at k moduli runs such passes: 32-bit ranks, pair passes left to the library.
-bool whole_size(const ofp_ctx* c, int n, int k) {
+// Whether n at k moduli is of that size, and whether it runs such passes: 32-bit ranks,
+// pair passes left to the library, room for more than the state.
+bool small_state(int n, int k) {
     uint64_t nm, nb;
-    return c->pair_rows < 0 && c->layout == 1 && c->index_bits != 64 && n >= 2 && n <= 22 && counts(n, &nm, &nb) &&
-           k <= kWholeKC && (nm + nb) * k < kWholeWords;
+    return n >= 2 && n <= 22 && counts(n, &nm, &nb) && k <= kWholeKC && (nm + nb) * k < kWholeWords;
+}
+bool whole_size(const ofp_ctx* c, int n, int k) {
+    return c->pair_rows < 0 && c->layout == 1 && c->index_bits != 64 && c->extra_memory && small_state(n, k);
 }
 bool whole_ready(const ofp_ctx* c, const Sweep& s) { return s.whole && s.layout == 1 && whole_size(c, s.n, s.K); }
 
+// Device bytes of s: its state, and what it holds beside it.
+uint64_t state_held(const Sweep& s) { return s.main_cap + s.blk_cap; }
+uint64_t extra_held(const Sweep& s) {
+    return s.main2_cap + s.blk2_cap + s.gscratch_cap + (uint64_t)s.mods_cap * (sizeof(uint32_t) + sizeof(uint64_t) * glue::kAccWords);
+}
+constexpr int kModsCap = 16;
+// The most that a solve of (n, k) in state-major layout holds beside its state.
+uint64_t extra_bytes(int n, int k) {
+    struct Host {
+        glue::Ballot b;
+        Host() { glue::build_ballot(b); }
+    };
+    static const Host host;
+    const int W = n + 1;
+    return (small_state(n, k) ? state_bytes(1, n, k) : 0) +
+           (W >= kHalfMinW && W <= glue::kSumStrands + 1 ? glue::scratch_need(host.b, W, k) : 0) +
+           (uint64_t)std::max(k, kModsCap) * (sizeof(uint32_t) + sizeof(uint64_t) * glue::kAccWords);
+}
+
+// Ensure device buffers of s for (n, moduli) in the context's current layout.
 ofp_status ensure_state(ofp_ctx* c, Sweep& s, int n, const uint32_t* moduli, int k) {
     uint64_t nm, nb;
     if (!counts(n, &nm, &nb)) return fail(c, OFP_E_RANGE, "n must be in 1..27");
@@ -382,6 +425,10 @@ ofp_status ensure_state(ofp_ctx* c, Sweep& s, int n, const uint32_t* moduli, int
         release_window(c);
         size_t fr = 0, tot = 0;
         OFP_HIP(c, hipMemGetInfo(&fr, &tot), "hipMemGetInfo");
+        if (mb + bb + c->reserve > fr && spare_bytes(c)) {
+            release_spare(c);
+            OFP_HIP(c, hipMemGetInfo(&fr, &tot), "hipMemGetInfo");
+        }
         if (mb + bb + c->reserve > fr)
             return fail(c, OFP_E_MEMORY, "insufficient HBM: need " + std::to_string(mb + bb) +
                                              " bytes, free " + std::to_string(fr));
@@ -404,13 +451,13 @@ ofp_status ensure_state(ofp_ctx* c, Sweep& s, int n, const uint32_t* moduli, int
             free_second(s);
         }
     }
-    if (s.mods_cap < k) {
+    if (s.mods_cap < k) {  // (extra_bytes counts these)
         sweep_free(s, s.mods_dev);
         sweep_free(s, s.acc);
         s.mods_dev = nullptr;
         s.acc = nullptr;
         s.mods_cap = 0;
-        const int cap = std::max(k, 16);
+        const int cap = std::max(k, kModsCap);
         OFP_HIP(c, sweep_alloc(s, (void**)&s.mods_dev, cap * sizeof(uint32_t)), "allocate moduli");
         OFP_HIP(c, sweep_alloc(s, (void**)&s.acc, cap * sizeof(uint64_t) * glue::kAccWords), "allocate sums");
         s.mods_cap = cap;
@@ -878,7 +925,8 @@ ofp_status enqueue_glue(ofp_ctx* c, Sweep& s, int* launches) {
 // reference residues).  Makes the lists of 19 strands and the scratch where the
 // width needs them; where those do not fit HBM the solve runs all rows.
 bool half_ready(ofp_ctx* c, Sweep& s) {
-    if (s.layout != 1 || cap_pct(c, s) <= 0 || s.row != 0 || s.W < 4 || s.W > glue::kSumStrands + 1 || !s.acc) return false;
+    if (s.layout != 1 || cap_pct(c, s) <= 0 || s.row != 0 || s.W < kHalfMinW || s.W > glue::kSumStrands + 1 || !s.acc)
+        return false;
     if (s.W > glue::kBaseStrands + 1 && !c->gtab[1].mem) {
         size_t fr = 0, tot = 0;
         // 2 bytes per open meander with 19 crossings: 16 MB
@@ -891,7 +939,7 @@ bool half_ready(ofp_ctx* c, Sweep& s) {
     }
     const size_t need = glue::scratch_need(c->ballot, s.W, s.Kp);
     if (need > s.gscratch_cap) {
-        if (s.fixed) return false;
+        if (s.fixed || !c->extra_memory) return false;
         sweep_free(s, s.gscratch);
         s.gscratch = nullptr;
         s.gscratch_cap = 0;
@@ -1349,8 +1397,8 @@ ofp_status ofp_plan(ofp_ctx* c, int n, int k, ofp_plan_info* out) {
     size_t fr = 0, tot = 0;
     OFP_HIP(c, hipSetDevice(c->device), "hipSetDevice");
     OFP_HIP(c, hipMemGetInfo(&fr, &tot), "hipMemGetInfo");
-    // memory already held by this context's own state can be reused
-    out->free_bytes = fr + c->st.main_cap + c->st.blk_cap + c->st.main2_cap + c->st.blk2_cap;
+    // memory already held by this context's own state can be reused, what it holds beside it given up
+    out->free_bytes = fr + state_held(c->st) + spare_bytes(c);
     out->fits = out->state_bytes + c->reserve <= out->free_bytes;
     return OFP_OK;
 }
@@ -1486,7 +1534,7 @@ ofp_status ofp_solve(ofp_ctx* c, int n, const uint32_t* moduli, int k, uint32_t*
     size_t fr = 0, tot = 0;
     OFP_HIP(c, hipSetDevice(c->device), "hipSetDevice");
     OFP_HIP(c, hipMemGetInfo(&fr, &tot), "hipMemGetInfo");
-    const uint64_t avail = fr + c->st.main_cap + c->st.blk_cap + c->st.main2_cap + c->st.blk2_cap + c->win_bytes + c->stage_bytes;
+    const uint64_t avail = fr + state_held(c->st) + spare_bytes(c) + c->win_bytes + c->stage_bytes;
     int g = c->max_batch > 0 ? std::min(k, c->max_batch) : k;
     while (g > 1 && state_bytes(c->layout, n, g) + c->reserve > avail) --g;
     if (state_bytes(c->layout, n, g) + c->reserve > avail)
@@ -1570,6 +1618,17 @@ ofp_status ofp_solve_static(ofp_ctx* c, int n, const uint32_t* moduli, int k, ui
     s.main = s.blk = s.main2 = s.blk2 = nullptr;
     s.main2_cap = s.blk2_cap = 0;
     return st;
+}
+
+ofp_status ofp_set_extra_memory(ofp_ctx* c, int on) {
+    if (!c) return OFP_E_ARG;
+    c->extra_memory = on != 0;
+    return OFP_OK;
+}
+
+uint64_t ofp_extra_bytes(int n, int k) {
+    uint64_t nm, nb;
+    return counts(n, &nm, &nb) && k >= 1 && k <= 1024 ? extra_bytes(n, k) : 0;
 }
 
 ofp_status ofp_set_max_batch(ofp_ctx* c, int max_moduli) {
@@ -2060,6 +2119,10 @@ ofp_status stage_buffer(ofp_ctx* c, size_t bytes, char** out) {
     }
     size_t fr = 0, tot = 0;
     OFP_HIP(c, hipMemGetInfo(&fr, &tot), "hipMemGetInfo");
+    if (bytes + c->reserve > fr && spare_bytes(c)) {
+        release_spare(c);
+        OFP_HIP(c, hipMemGetInfo(&fr, &tot), "hipMemGetInfo");
+    }
     if (bytes + c->reserve > fr) return fail(c, OFP_E_MEMORY, "exchange staging does not fit HBM beside the window");
     const size_t slack = bytes + c->reserve + bytes / 16 <= fr ? bytes / 16 / 256 * 256 : 0;  // as the window's
     OFP_HIP(c, hipMalloc(&c->stage, bytes + slack), "exchange buffer");
@@ -2345,7 +2408,7 @@ ofp_status ofp_job_info_get(ofp_job* j, ofp_job_info* info) {
     info->rows_total = j->sw.W;
     info->rows_enqueued = j->rows_enqueued;
     info->idle = (q == hipSuccess) ? 1 : 0;
-    info->state_bytes = j->sw.main_cap + j->sw.blk_cap;
+    info->state_bytes = state_held(j->sw) + extra_held(j->sw);
     info->transitions_per_row = (uint64_t)(j->sw.W - 1) * (j->sw.nmain + j->sw.nblk) * (uint64_t)j->sw.K;
     return OFP_OK;
 }

@@ -31,7 +31,7 @@ EXPORTS = (
     "ofp_shard_plan", "ofp_shard_sweep", "ofp_group_plan", "ofp_group_sweep", "ofp_set_height_caps", "ofp_height_cap", "ofp_set_xcd_pieces",
     "ofp_set_sorted_cells", "ofp_time_cells", "ofp_set_index_width", "ofp_set_max_batch",
     "ofp_moduli_groups", "ofp_solve_static", "ofp_set_pair_passes", "ofp_group_exchange",
-    "ofp_set_group_launch",
+    "ofp_set_group_launch", "ofp_set_extra_memory", "ofp_extra_bytes",
 )
 
 
@@ -212,6 +212,8 @@ def load() -> ctypes.CDLL:
                                             ctypes.c_int]),
         "ofp_set_index_width": (ctypes.c_int32, [vp, ctypes.c_int]),
         "ofp_set_max_batch": (ctypes.c_int32, [vp, ctypes.c_int]),
+        "ofp_set_extra_memory": (ctypes.c_int32, [vp, ctypes.c_int]),
+        "ofp_extra_bytes": (ctypes.c_uint64, [ctypes.c_int, ctypes.c_int]),
         "ofp_set_pair_passes": (ctypes.c_int32, [vp, ctypes.c_int, ctypes.c_uint32]),
         "ofp_set_group_launch": (ctypes.c_int32, [vp, ctypes.c_int, ctypes.c_longlong]),
         "ofp_solve_static": (ctypes.c_int32, [vp, ctypes.c_int, u32p, ctypes.c_int, u32p]),
@@ -266,6 +268,12 @@ def state_counts(n: int) -> tuple[int, int]:
 
 
 DEFAULT_CAP_PERCENT = 85
+
+
+def extra_bytes(n: int, k: int) -> int:
+    """The most that a solve or job of (n, k) holds beside its state (host computation,
+    no GPU needed)."""
+    return load().ofp_extra_bytes(n, k)
 
 
 def moduli_groups(k: int, max_per_sweep: int) -> list[int]:
@@ -426,6 +434,11 @@ class Context:
     def set_max_batch(self, max_moduli: int) -> None:
         """At most max_moduli moduli per sweep of solve() (0 = as many as fit HBM)."""
         self._check(self._lib.ofp_set_max_batch(self._h, max_moduli), "ofp_set_max_batch")
+
+    def set_extra_memory(self, on: bool) -> None:
+        """Whether solves and jobs may hold more than their state where that makes them
+        faster (extra_bytes); on by default."""
+        self._check(self._lib.ofp_set_extra_memory(self._h, 1 if on else 0), "ofp_set_extra_memory")
 
     def set_launch(self, threads: int, blocks_per_cu: int) -> None:
         self._check(self._lib.ofp_set_launch(self._h, threads, blocks_per_cu), "ofp_set_launch")

@@ -5,10 +5,12 @@ frontier state resident on the device as a job (ofp.Job: its own stream,
 its own interleaved state) and
 
   * admits pending work whenever a job slot and HBM are free, using the
-    state-size model (bytes = (main + blocked states) x padded k x 4, the same
-    figure as ofp_plan) against a fixed budget (free HBM at start minus the
-    reserve) -- the reference's admission test is its HBM budget check
-    (row6crt20.cu:1751-1755);
+    state-size model (bytes = (main + blocked states) x k x 4, the same
+    figure as ofp_plan, and what the job holds beside its state, ofp_extra_bytes)
+    against a fixed budget (free HBM at start minus the reserve) -- the
+    reference's admission test is its HBM budget check (row6crt20.cu:1751-1755).
+    A job whose state alone fits the budget runs alone with nothing beside it;
+    one that the device still has no room for waits for another to retire;
   * batches at admission: all pending requests with the same n are merged into
     ONE job whose moduli are the union of theirs (duplicates shared), up to 16
     moduli (one cell launch), so their residues ride in one interleaved sweep;
@@ -64,8 +66,7 @@ class _Active:
 def state_bytes(n: int, k: int, layout: int = 1) -> int:
     nm, nb = _lib.state_counts(n)
     pad = lambda x: (x + 63) // 64 * 64  # noqa: E731
-    kp = (k + 1) // 2 * 2 if (layout == 1 and k > 1) else k
-    return (pad(nm) + pad(nb)) * kp * 4
+    return (pad(nm) + pad(nb)) * k * 4
 
 
 def poisson_stream(count: int, rate: float, seed: int, n_lo: int = 14, n_hi: int = 21,
@@ -101,6 +102,10 @@ class Server:
     def submit(self, req: Request) -> None:
         self.pending.append(req)
 
+    def _extra_memory(self, on: bool) -> None:
+        if self.ctx is not None:  # (a scheduler under test has no device)
+            self.ctx.set_extra_memory(on)
+
     def _admit(self, now: float) -> None:
         while self.pending and len(self.active) < self.max_jobs:
             head = self.pending[0]
@@ -117,12 +122,24 @@ class Server:
             need = state_bytes(head.n, len(mods))
             if need > self.budget_bytes:
                 raise RuntimeError(f"request n={head.n} k={len(mods)} needs {need} bytes > budget")
-            if self.used_bytes + need > self.budget_bytes:
-                return  # wait for memory: admission is FIFO on the head request
+            extra = _lib.extra_bytes(head.n, len(mods))
+            if self.used_bytes + need + extra > self.budget_bytes:
+                if self.active:
+                    return  # wait for memory: admission is FIFO on the head request
+                extra = 0
+            need += extra
             if self.tuned:
                 autotune.apply(self.ctx, head.n, len(mods))
-            job = _lib.Job(self.ctx, head.n, mods)
-            job.enqueue(head.n + 1)  # all W rows, asynchronously on the job's stream
+            try:
+                self._extra_memory(extra > 0)
+                job = _lib.Job(self.ctx, head.n, mods)
+                job.enqueue(head.n + 1)  # all W rows, asynchronously on the job's stream
+            except _lib.OfpError as e:
+                if e.status != _lib.OFP_E_MEMORY or not self.active:
+                    raise
+                return  # the device has less than the budget says: wait for a job to retire
+            finally:
+                self._extra_memory(True)
             for r in group:
                 self.pending.remove(r)
                 r.job_moduli = len(mods)
