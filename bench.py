@@ -462,19 +462,17 @@ def main() -> int:
             with ofp.Context(device=0) as c:
                 autotune.apply(c, ns, 1)
                 c.solve(ns, [PRIMES[0]])
-                times, res = [], None
+                times, res, st = [], None, None
                 for _ in range(3):
                     t0s = time.perf_counter()
-                    r, _ = c.solve(ns, [PRIMES[0]])
+                    r, st = c.solve(ns, [PRIMES[0]])
                     times.append(time.perf_counter() - t0s)
                     res = r[0]
             med = sorted(times)[1]
-            Ws = ns + 1
-            Ss = sum(ofp.state_counts(ns))
             want = GOLDEN_FIRST.get(ns)
             small[f"n{ns}"] = {"solve_s": med, "residue": res, "modulus": PRIMES[0],
                                "verified": (res == want[1]) if want and want[0] == PRIMES[0] else None,
-                               "transitions_per_s": Ws * (Ws - 1) * Ss / med,
+                               "transitions_per_s": st["transitions"] / med,
                                "residues_per_hour": 3600.0 / med}
             log(f"bench: plain n={ns} solve {med * 1e3:.1f} ms, residue {res}")
 

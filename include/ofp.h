@@ -55,7 +55,7 @@ typedef struct ofp_plan_info {
     uint64_t main_states;     /* H_DP[W][1] = M_{n+2} - M_{n+1}  (row6crt20.cu:1748) */
     uint64_t blocked_states;  /* H_DP[W-1][1] */
     uint64_t state_bytes;     /* device bytes of the interleaved state for k moduli */
-    uint64_t transitions;     /* W*(W-1)*(main+blocked)*k: frontier transitions per solve */
+    uint64_t transitions;     /* W*(W-1)*(main+blocked)*k: frontier transitions of all rows */
     uint64_t free_bytes;      /* free HBM on the device right now, and what the context would give up */
     int fits;                 /* state_bytes + reserve <= free_bytes */
 } ofp_plan_info;
@@ -63,11 +63,16 @@ typedef struct ofp_plan_info {
 typedef struct ofp_stats {
     double wall_s;            /* whole solve, host clock */
     double kernel_s;          /* sum of cell-kernel time (HIP events), 0 if not timed */
-    uint64_t transitions;     /* frontier transitions performed */
+    /* frontier transitions performed: cells applied x (main+blocked) x k, a
+     * height-capped cell counting like any other.  A solve from half of its rows
+     * (ofp_solve and jobs with height caps on, n = 3..23) applies half of the cells. */
+    uint64_t transitions;
     uint64_t main_states, blocked_states;
-    int rows, cells_per_row, launches;
+    int rows;                 /* rows the state has advanced: W per sweep of a solve */
+    int cells_per_row, launches;
     /* kernel time split: runs of rows whose cells all sweep the full state
-     * (full_*) and rows with height-capped cells (capped_*) */
+     * (full_*) and rows with height-capped cells (capped_*); the step that ends a
+     * solve from half of its rows is in neither, only in kernel_s and launches */
     double full_kernel_s, capped_kernel_s;
     int full_launches, capped_launches;
 } ofp_stats;

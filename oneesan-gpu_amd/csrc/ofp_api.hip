@@ -1437,7 +1437,9 @@ static ofp_status row_sweep(ofp_ctx* c, int rows, ofp_stats* st, bool half) {
         st->rows = rows;
         st->cells_per_row = s.W - 1;
         st->launches = launches;
-        st->transitions = (uint64_t)rows * (s.W - 1) * (s.nmain + s.nblk) * (uint64_t)s.K;
+        // half: W/2 rows and, odd W, the upper half of the middle one's cells
+        const uint64_t cells = half ? (uint64_t)s.W * (s.W - 1) / 2 : (uint64_t)rows * (s.W - 1);
+        st->transitions = cells * (s.nmain + s.nblk) * (uint64_t)s.K;
     }
     return OFP_OK;
 }
