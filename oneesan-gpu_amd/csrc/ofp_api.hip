@@ -1886,7 +1886,10 @@ ofp_status ofp_group_sweep(ofp_ctx* c, const ofp_group_spec* sp, ofp_group_info*
     std::vector<uint64_t> ccount((size_t)G * npairs * 5, 0);
     if (npairs) {
         static uint64_t fm[kDpRows][kDpCols];
-        static cell::Pair<uint32_t> t[kDpRows][kDpCols];
+        // in the columns the kernels read, as class_table_bytes counts them
+        constexpr int kCols = cell::LdsCols<uint32_t>::value;
+        static cell::Pair<uint32_t> t[kDpRows][kCols];
+        static_assert(sizeof t >= sizeof(cell::Pair<uint32_t>) * cell::kLdsRows * kCols, "a packed class table");
         for (uint32_t g = 0; g < G; ++g) {
             cell::Occupancy om, ob;
             cell::group_occupancy(sp->high != 0, W, L, sp->first_group + g, om, ob);
@@ -1897,7 +1900,7 @@ ofp_status ofp_group_sweep(ofp_ctx* c, const ofp_group_spec* sp, ofp_group_info*
                 const int p = x & 0xff;
                 for (int di = 0; di < 5; ++di) {
                     const size_t slot = ((size_t)g * npairs + j) * 5 + di;
-                    pair::pack_group_class_table<uint32_t, kDpCols>(om, fm, p, kPairD[di], t);
+                    pair::pack_group_class_table<uint32_t, kCols>(om, fm, p, kPairD[di], t);
                     std::memcpy(cts.data() + slot * ctb, t, ctb);
                     ccount[slot] = pair::group_class_count(om, fm, W, p, kPairD[di]);
                 }
