@@ -18,19 +18,19 @@ Measured in one process, in this order:
     rows of work.
   * steps (the `value`): --warmup untimed and --steps timed row sweeps of the
     same state with height caps off, so that every row does its full
-    algorithmic work (W-1 cells x S states x k moduli transitions); each cell is
-    launched on its own between HIP events on the library's stream, and the
+    algorithmic work (W-1 cells x S states x k moduli transitions); each cell or
+    pair pass (two cells) is timed between HIP events on the library's stream, and the
     timed region is bracketed by device synchronisation.  value = transitions
     of the timed rows / their wall time.
-  * roofline: per kernel (cell_sorted_kernel: cells p >= 6, cell_kernel: p <= 5)
-    the mean launch duration over the timed rows' events; declared algorithmic
-    bytes per launch = 8 B x k x S (one 4-byte read and one 4-byte write per
+  * roofline: per kernel (pair_kernel; cell kernels where a cell runs alone)
+    the mean duration of a pass or launch over the timed rows' events; declared
+    algorithmic bytes per pass or launch = 8 B x k x S (one 4-byte read and one 4-byte write per
     state per modulus).  `roofline` is the dominant kernel's.  HBM traffic per
     launch is measured before the GPU work starts, by running one row of the same
     configuration in a child process under rocprofv3 with the DRAM request
     counters TCC_EA0_RDREQ_DRAM_32B and TCC_EA0_WRREQ_WRITE_DRAM_32B (32-byte
     units; no calibration needed); null if rocprofv3 is unavailable.  The
-    height-capped kernel of the solve is reported beside them.
+    height-capped rows of the solve are reported beside them.
   * plain: the same solve with k=1 (one residue at a time), timed whole ->
     residues/hour of the plain form, and its per-kernel launch times.
   * plain_small: whole one-modulus solves at n=12 and n=18 (median of three).

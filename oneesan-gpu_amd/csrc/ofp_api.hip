@@ -609,8 +609,9 @@ bool pair_ready(const ofp_ctx* c, const Sweep& s) { return pairs_apply(c, s.n) &
 // p_hi - p, kind 2) gets its time and the second an empty interval (kind 3).
 // The library's default pairing: every pair except cells 3 and 2 (n=21 at 13 moduli
 // 50.9 ms, with cell 1 alone 75.3; cell 3 alone and 2, 1 65.3) and, from 2 to 7 moduli, cells 4
-// and 3 (n=20 at 4 6.2 against 2.7 + 2.9 ms; at 11 13.4 against 6.9 + 7.2, n=18 at one 0.28
-// against 0.19 + 0.19).  The other passes are 1.05-1.9x faster than their two cells.
+// and 3 (ms of the pass and of its two cells, n=20 at 2 moduli 4.46, 3.64; at 4 6.21, 5.54; 5 8.69,
+// 6.85; 6 9.12, 8.16; 7 10.11, 9.46; 8 9.77, 10.25; 9 12.25, 12.11; 10 12.54, 12.86; n=18 at one 0.28,
+// 0.38).  The other passes are 1.05-1.9x faster than their two cells.
 uint32_t default_pair_mask(int kc) { return ~((1u << 3) | (kc > 1 && kc < 8 ? 1u << 4 : 0u)); }
 // Group sweeps (4 moduli, n=27 windows over three streams): pair passes over
 // every pair of cells from 7 up; cells 6..1 one per launch, where the pair
@@ -1079,8 +1080,8 @@ int moduli_groups(int k, int g, int* sizes, int cap) {
 }
 
 // Residues between a caller's state-major array (n states of k) and device words in a
-// layout with stride Kp.  Equal strides (k = 1 or even, state-major) copy at once;
-// others go through a device buffer of at most kIoBytes, where a kernel changes the
+// layout with stride Kp.  Equal strides, state-major, copy at once (full states always,
+// windows of one or an even count of moduli); others go through a device buffer of at most kIoBytes, where a kernel changes the
 // stride, so the host never touches single residues.
 constexpr size_t kIoBytes = 64ull << 20;
 ofp_status io_buffer(ofp_ctx* c, size_t bytes, uint32_t** out) {

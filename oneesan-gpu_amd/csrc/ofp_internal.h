@@ -48,9 +48,9 @@ __host__ __device__ inline uint64_t state_elem(int layout, uint64_t i, int K, in
     return layout == 0 ? aosoa(i, K, j) : i * (uint64_t)K + (uint64_t)j;
 }
 // Interleave stride of a full-state sweep: a record is its k residues, so an odd count
-// moves no padding (a stride rounded up to even: an n=21 row at 13 moduli 307 against
-// 280 ms, an n=20 solve at 11 789 against 739 ms).  Windows of shard and group sweeps and the exchange's records
-// keep an even stride (window_stride): the exchange moves two residues per access.
+// moves no padding (with a stride rounded up to even an n=20 solve at 11 moduli took 789
+// against 739 ms).  Windows of shard and group sweeps and the exchange's records keep an
+// even stride (window_stride): the exchange moves two residues per access.
 inline int interleave_stride(int, int k) { return k; }
 inline int window_stride(int k) { return k > 1 ? (k + 1) / 2 * 2 : k; }
 
